@@ -72,11 +72,8 @@ namespace {
 #ifndef EVS_GATHER_STORE_SC1
 #define EVS_GATHER_STORE_SC1 1
 #endif
-// Word order in a tile, per direction. 0: along the cache in the common layouts (a wave covers
+// The scatter's word order in a tile. 0: along the cache in the common layouts (a wave covers
 // consecutive heads of one slot, K then V); 1: along the staging buffer (whole staged rows).
-#ifndef EVS_GATHER_ORDER
-#define EVS_GATHER_ORDER 1
-#endif
 #ifndef EVS_SCATTER_ORDER
 #define EVS_SCATTER_ORDER 1
 #endif
@@ -185,7 +182,8 @@ constexpr int nt_of(int d, int i) {
          : d == kGather    ? EVS_GATHER_NT
                            : EVS_SCATTER_NT;
 }
-constexpr int order_of(int d) { return d == kGather ? EVS_GATHER_ORDER : EVS_SCATTER_ORDER; }
+// the gather's words run along the staging buffer, so that its tile's words are all live ones
+constexpr int order_of(int d) { return d == kGather ? 1 : EVS_SCATTER_ORDER; }
 constexpr int word_order(int d, int i) { return i == kByPairs ? EVS_PAIRS_ORDER : order_of(d); }
 static_assert(threads_of(kGather, kBySlots) >= kMaxTileSlots &&
                   threads_of(kScatter, kBySlots) >= kMaxTileSlots &&
@@ -193,26 +191,6 @@ static_assert(threads_of(kGather, kBySlots) >= kMaxTileSlots &&
               "the first TS threads fill a tile's slot offsets: a workgroup needs kMaxTileSlots");
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-// one cell per word of a pass, at the widest pass
-constexpr int kSinkWords = 1024;
-static_assert(threads_of(kGather, kBySlots) * vpt_of(kGather, kBySlots) <= kSinkWords &&
-                  threads_of(kScatter, kBySlots) * vpt_of(kScatter, kBySlots) <= kSinkWords &&
-                  threads_of(kScatter, kByPairs) * vpt_of(kScatter, kByPairs) <= kSinkWords,
-              "the sink holds one cell per word of a pass");
-
-// Where a gathered word that moves nothing goes: a lane with no word (a slot past n, a word past
-// the tile) loads from and stores into its own 16-byte cell here instead of branching around the
-// access. With no branch between them, a thread's loads are all issued before its first store and
-// each store waits only for its own data; a branch around each access makes the compiler wait for
-// every memory operation in flight before each store, which serialises a thread's stores (the
-// gather measured 1 % faster without). The scatter keeps the branches: its scattered stores ran
-// 0.5-1.5 % faster serialised than all in flight. The contents are never read as data.
-// Workgroups take one of kSinkCopies regions by id: with one region shared by all, a call whose
-// tiles leave most lanes idle (a decode step of 1-4 slots) sent every such store to the same
-// 16 KiB, and so to the same few memory channels, and took 4.5 us where 8 slots took 2.45.
-constexpr int kSinkCopies = 64;
-__device__ u32x4 g_sink[kSinkCopies * kSinkWords];
 
 struct RowsArgs {
   const int64_t* layer_ptrs;  // device: each layer's cache base address
@@ -237,10 +215,11 @@ struct RowsArgs {
   int TS;                     // slots per tile
   int group_fastest;          // tile numbers run through head groups first
   int xcd_chunk;              // tiles per XCD per run (see xcd_tile)
-  uint32_t tile_words;        // TS * HG * 2 * W
+  uint32_t W;                 // words per half-row
   FastDiv div_w;              // words per half-row
   FastDiv div_h;              // heads per tile
   FastDiv div_ts;             // slots per tile
+  FastDiv div_ts_last;        // slots of a layer's last tile
   FastDiv div_tiles;          // slot tiles per (layer, head group)
   FastDiv div_groups;         // head groups
 };
@@ -401,24 +380,25 @@ __device__ __forceinline__ int64_t slot_offset(const RowsArgs& a, uint32_t layer
 }
 
 // Where word v of a tile lies: head index h within the tile's group, slot tl within the tile,
-// K or V (k) and word j of the half-row.
+// K or V (k) and word j of the half-row. The tile's own slot count (a layer's last tile may have
+// fewer than TS) divides the words, so a tile's live words are exactly [0, words).
 struct WordAt {
   uint32_t h, tl, k, j;
 };
 
 template <int kOrder>
-__device__ __forceinline__ WordAt word_at(const RowsArgs& a, uint32_t v) {
+__device__ __forceinline__ WordAt word_at(const RowsArgs& a, const FastDiv& div_ts, uint32_t v) {
   WordAt w;
   uint32_t q, q2;
   a.div_w.divmod(v, q, w.j);
   if (kOrder == 0) {
     // v = ((k * TS + tl) * HG + h) * W + j
     a.div_h.divmod(q, q2, w.h);
-    a.div_ts.divmod(q2, w.k, w.tl);
+    div_ts.divmod(q2, w.k, w.tl);
   } else {
     // v = ((h * TS + tl) * 2 + k) * W + j: K then V of one staged row, row after row
     w.k = q & 1u;
-    a.div_ts.divmod(q >> 1, w.h, w.tl);
+    div_ts.divmod(q >> 1, w.h, w.tl);
   }
   return w;
 }
@@ -431,55 +411,94 @@ __device__ __forceinline__ int64_t staged_offset(const RowsArgs& a, uint32_t h0,
 }
 
 // Move one tile's words: the slots' offsets and the heads' are in LDS, and for the pair scatter
-// the staged rows'.
+// the staged rows'. A wave past the tile's last word leaves; in the wave that holds the last word
+// the gather's lanes past it move that word again, which costs nothing (the same lines in the
+// same instruction) and keeps every access free of a branch: with a branch around each, the
+// compiler waits for every memory operation in flight before each store, which serialises a
+// thread's stores (1 % slower on a full tile). Before, lanes without a word moved a cell of a
+// device array of their own instead: where the head dim leaves a tile's passes partly empty, those
+// write-through stores of every workgroup met on the same few lines and held the gather to
+// 1.5-1.8 TB/s. 400 MB of one or eight heads, head dims 80, 96, 112, 120 and 192 in bf16 and fp8:
+// 1,461-1,813 GB/s before, 5,076-6,105 now (bf16 120, eight heads kv_first 1,483 and 5,078; 112
+// combined 1,650 and 5,678); head dim 128 unchanged (5,642 and 5,613; one head 6,103 and 6,105).
+// The scatter keeps a branch around each access: its scattered stores ran 0.5-1.5 %
+// faster serialised than all in flight.
 template <typename T, int D, int I>
 __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_slot,
                                           const int64_t* s_head, const int64_t* s_src,
                                           int64_t layer_base, uint32_t layer, uint32_t group,
                                           int64_t t0) {
+  constexpr int kThreads = threads_of(D, I);
+  constexpr int kVpt = vpt_of(D, I);
+  constexpr int kOrder = word_order(D, I);
   const uint32_t h0 = group * a.HG;
-  const int tid = threadIdx.x;
+  const uint32_t tid = threadIdx.x;
   char* cache_w = reinterpret_cast<char*>(layer_base);
   char* rows_l = a.rows + static_cast<int64_t>(layer) * a.H * a.cap * (2 * a.half_bytes);
 
-  constexpr int kThreads = threads_of(D, I);
-  char* sink = reinterpret_cast<char*>(g_sink + (blockIdx.x % kSinkCopies) * kSinkWords) +
-               tid * sizeof(u32x4);
-  constexpr int kVpt = vpt_of(D, I);
-  for (uint32_t v0 = 0; v0 < a.tile_words; v0 += kThreads * kVpt) {
-    T w[kVpt];
-    const char* src[kVpt];
-    char* dst[kVpt];
-    bool live[kVpt];
-#pragma unroll
-    for (int i = 0; i < kVpt; i++) {
-      const uint32_t v = v0 + i * kThreads + tid;
-      const WordAt at = word_at<word_order(D, I)>(a, v);
-      const bool in_tile = v < a.tile_words && h0 + at.h < static_cast<uint32_t>(a.H);
-      const int64_t slot_off = in_tile ? s_slot[at.tl] : -1;
-      char* cache = cache_w + slot_off + s_head[in_tile ? at.h : 0] + at.k * a.skv + at.j * a.sj;
-      const int64_t row = I == kByPairs ? s_src[at.tl] : t0 + at.tl;
-      char* staged = rows_l + staged_offset(a, h0, row, at, sizeof(T));
-      char* cell = sink + i * kThreads * sizeof(u32x4);
-      live[i] = slot_off >= 0;
-      src[i] = live[i] ? (D == kGather ? cache : staged) : cell;
-      dst[i] = live[i] ? (D == kGather ? staged : cache) : cell;
-    }
+  const bool whole = t0 + a.TS <= a.n;
+  const uint32_t slots = whole ? a.TS : static_cast<uint32_t>(a.n - t0);
+  const FastDiv div_ts = whole ? a.div_ts : a.div_ts_last;
+  // in the cache's word order the heads run inside a slot, so a last group's missing heads stay
+  // among the words (and move nothing)
+  const uint32_t heads = kOrder == 1 && h0 + a.HG > static_cast<uint32_t>(a.H) ? a.H - h0 : a.HG;
+  const uint32_t words = heads * slots * 2 * a.W;
+
+  const auto locate = [&](uint32_t v, char*& cache, char*& staged) {
+    const WordAt at = word_at<kOrder>(a, div_ts, v);
+    const int64_t slot_off = s_slot[at.tl];
+    const int64_t row = I == kByPairs ? s_src[at.tl] : t0 + at.tl;
+    cache = cache_w + slot_off + s_head[at.h] + at.k * a.skv + at.j * a.sj;
+    staged = rows_l + staged_offset(a, h0, row, at, sizeof(T));
+    return slot_off >= 0 && (kOrder == 1 || h0 + at.h < static_cast<uint32_t>(a.H));
+  };
+
+  for (uint32_t v0 = 0; v0 < words; v0 += kThreads * kVpt) {
     if (D == kGather) {
-      // Each load stays where it is issued (the scheduler otherwise issued the second word's
-      // load first, after the first's address work, so the first store waited for both loads):
-      // now the first word's store waits for its own load only. 9-11 interleaved rounds on two
-      // boxes: C2 6,110-6,113 against 6,096-6,098 GB/s, C3 6,159 against 6,124, one bf16 head
-      // 6,266 against 6,197, the combined layout 6,090 against 6,057, blocks_first unchanged.
+      const uint32_t wave = v0 + __builtin_amdgcn_readfirstlane(tid & ~63u);
+      if (wave >= words) break;  // this wave's later passes lie further on still
+      if (wave + (kVpt - 1) * kThreads < words) {
+        T w[kVpt];
+        char* src[kVpt];
+        char* dst[kVpt];
+#pragma unroll
+        for (int i = 0; i < kVpt; i++) {
+          const uint32_t v = v0 + i * kThreads + tid;
+          locate(i == kVpt - 1 && v >= words ? words - 1 : v, src[i], dst[i]);
+        }
+        // Each load stays where it is issued (the scheduler otherwise issued the second word's
+        // load first, after the first's address work, so the first store waited for both loads):
+        // now the first word's store waits for its own load only. 9-11 interleaved rounds on two
+        // boxes: C2 6,110-6,113 against 6,096-6,098 GB/s, C3 6,159 against 6,124, one bf16 head
+        // 6,266 against 6,197, the combined layout 6,090 against 6,057, blocks_first unchanged.
+#pragma unroll
+        for (int i = 0; i < kVpt; i++) {
+          w[i] = load_word<T, (nt_of(D, I) & 1) != 0>(src[i]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < kVpt; i++)
+          store_word<T, (nt_of(D, I) & 2) != 0, EVS_GATHER_STORE_SC1 != 0>(dst[i], w[i]);
+      } else {
+        // a pass that the tile does not fill: its words one at a time
+        for (uint32_t v1 = v0; v1 + (wave - v0) < words; v1 += kThreads) {
+          const uint32_t v = v1 + tid;
+          char *src, *dst;
+          locate(v < words ? v : words - 1, src, dst);
+          store_word<T, (nt_of(D, I) & 2) != 0, EVS_GATHER_STORE_SC1 != 0>(
+              dst, load_word<T, (nt_of(D, I) & 1) != 0>(src));
+        }
+      }
+    } else {
+      T w[kVpt];
+      char* src[kVpt];
+      char* dst[kVpt];
+      bool live[kVpt];
 #pragma unroll
       for (int i = 0; i < kVpt; i++) {
-        w[i] = load_word<T, (nt_of(D, I) & 1) != 0>(src[i]);
-        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t v = v0 + i * kThreads + tid;
+        live[i] = locate(v < words ? v : words - 1, dst[i], src[i]) && v < words;
       }
-#pragma unroll
-      for (int i = 0; i < kVpt; i++)
-        store_word<T, (nt_of(D, I) & 2) != 0, EVS_GATHER_STORE_SC1 != 0>(dst[i], w[i]);
-    } else {
 #pragma unroll
       for (int i = 0; i < kVpt; i++)
         if (live[i]) w[i] = load_word<T, (nt_of(D, I) & 1) != 0>(src[i]);
@@ -593,10 +612,11 @@ int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const ch
               "%s: %lld workgroups of %d threads exceed the launch limit of 2^32 - 1 work-items; "
               "split the call by layers", name, static_cast<long long>(grid), threads_of(D, I));
   a.TS = static_cast<int>(ts);
-  a.tile_words = static_cast<uint32_t>(ts * per_slot);
+  a.W = W;
   a.div_w = FastDiv(W);
   a.div_h = FastDiv(static_cast<uint32_t>(a.HG));
   a.div_ts = FastDiv(static_cast<uint32_t>(ts));
+  a.div_ts_last = FastDiv(static_cast<uint32_t>(a.n - (tiles - 1) * ts));
   a.div_tiles = FastDiv(static_cast<uint32_t>(tiles));
   a.div_groups = FastDiv(static_cast<uint32_t>(groups));
   hipLaunchKernelGGL((move_rows<T, D, I>), dim3(static_cast<uint32_t>(grid)),

@@ -57,6 +57,27 @@ def test_ragged_counts_leave_the_rows_past_n_alone(ext, layout, d, n):
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("d", [80, 96, 112, 120, 192, 1056])
+@pytest.mark.parametrize("n", [1, 8, 26])
+def test_passes_a_tile_does_not_fill(ext, layout, dtype, d, n):
+    """Head dims whose tiles leave lanes, or whole waves, of a pass without a word (1056 leaves a
+    second pass partly empty), at slot counts of one short tile, whole tiles and a last short one;
+    the rows past n and the spare capacity keep their bytes."""
+    layers = caches(layout, d, dtype, n_layers=L, nb=NB, h=H, seed=d + n)
+    slots, heads, cap, e = ragged_slots(n, n), [1, 2, 0], n + 3, layers[0].element_size()
+    want = np.full((L, len(heads), cap, 2, d), SENTINEL & (0xFF if e == 1 else 0xFFFF),
+                   dtype=np.uint8 if e == 1 else np.uint16)
+    out = torch.from_numpy(want.view(np.uint8).copy()).cuda()
+    oracle.gather_rows(layers, slots, heads, cap, d, BS, strides_of(layers[0]), e, out=want)
+    gpu = [t.cuda() for t in layers]
+    ext.gather_rows(ptrs(gpu), dev_long(slots), dev_long(heads), out.data_ptr(), cap, d, BS,
+                    list(strides_of(gpu[0])), e)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy().view(want.dtype), want)
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("blocks", [[3], [9, 0, 77], list(range(40, 57))])
 def test_ragged_block_lists(ext, layout, blocks):
     d = 8
