@@ -10,9 +10,9 @@
 // One workgroup owns a tile: its first TS threads turn the tile's slot ids (or block ids) into
 // byte offsets inside a layer, the first HG threads the head slots, both into LDS, so each moved
 // word costs two LDS reads and no 64-bit division. Each thread then moves VPT words at a time,
-// every load in flight before the first store. A word is 16 bytes when every half-row is
-// contiguous and 16-byte aligned on both sides (bf16 d=128: 16 words a half-row, fp8 d=128: 8),
-// else one element. Within a tile the words run along the staging buffer (K then V of one row,
+// every load in flight before the first store. A word is the widest of 16, 8, 4, 2 and 1 bytes
+// that every half-row, contiguous and aligned on both sides, is whole words of (bf16 d=128: 16
+// words of 16 bytes a half-row, fp8 d=120: 15 of 8), at least one element. Within a tile the words run along the staging buffer (K then V of one row,
 // row after row), so a wave stores whole rows: 1 KiB contiguous for bf16 d=128. For the gather
 // the tile numbers run through a slot range's head groups first, so the workgroups reading the
 // heads of one cache block (adjacent in every paged layout) are neighbours, dealt round-robin to
@@ -160,6 +160,8 @@ constexpr uint32_t kXcds = 8;
 #define EVS_RANGES_GROUP_FASTEST EVS_SCATTER_GROUP_FASTEST
 #endif
 
+// s_waitcnt's operand for vmcnt(0) alone: the other counters at their largest
+constexpr int kVmcntZero = 0x0f70;
 constexpr int kMaxTileSlots = 64;
 constexpr int kMaxHeads = 256;      // LDS table of head offsets
 
@@ -173,8 +175,14 @@ enum Index : int { kBySlots = 0, kByBlocks = 1, kByPairs = 2, kByRanges = 3 };
 constexpr int threads_of(int d, int i) {
   return i == kByPairs ? EVS_PAIRS_THREADS : d == kGather ? EVS_GATHER_THREADS : EVS_SCATTER_THREADS;
 }
-constexpr int vpt_of(int d, int i) {
-  return i == kByPairs ? EVS_PAIRS_VPT : d == kGather ? EVS_GATHER_VPT : EVS_SCATTER_VPT;
+// A narrower word's passes and tiles hold more of them: 2x at 8 bytes (the same bytes a tile), 4x
+// below, where the work is the address arithmetic a word takes. 400 MB gathered from one head, 4x
+// and 2x against 1x: 8-byte words (bf16 100) 5,507 and 5,467 against 3,670 GB/s, 2-byte words
+// (fp8 126) 3,433 and 2,428 against 1,546; (bf16 124, 8-byte) 4,286 and 5,516 against 4,560.
+constexpr int narrow_of(size_t word) { return word == 16 ? 1 : word == 8 ? 2 : 4; }
+constexpr int vpt_of(int d, int i, size_t word) {
+  return narrow_of(word) *
+         (i == kByPairs ? EVS_PAIRS_VPT : d == kGather ? EVS_GATHER_VPT : EVS_SCATTER_VPT);
 }
 constexpr int nt_of(int d, int i) {
   return i == kByPairs    ? EVS_PAIRS_NT
@@ -191,6 +199,7 @@ static_assert(threads_of(kGather, kBySlots) >= kMaxTileSlots &&
               "the first TS threads fill a tile's slot offsets: a workgroup needs kMaxTileSlots");
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 struct RowsArgs {
   const int64_t* layer_ptrs;  // device: each layer's cache base address
@@ -248,6 +257,8 @@ __device__ __forceinline__ void store_word(char* p, T v) {
     // s_nop gives that wait state whatever is scheduled next.
     asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 0" : : "v"(g), "v"(v)
                  : "memory");
+  else if constexpr (kNt && kSc1 && sizeof(T) == 8)
+    asm volatile("global_store_dwordx2 %0, %1, off sc1 nt" : : "v"(g), "v"(v) : "memory");
   else if (kNt)
     __builtin_nontemporal_store(v, g);
   else
@@ -380,8 +391,7 @@ __device__ __forceinline__ int64_t slot_offset(const RowsArgs& a, uint32_t layer
 }
 
 // Where word v of a tile lies: head index h within the tile's group, slot tl within the tile,
-// K or V (k) and word j of the half-row. The tile's own slot count (a layer's last tile may have
-// fewer than TS) divides the words, so a tile's live words are exactly [0, words).
+// K or V (k) and word j of the half-row. div_ts divides by the slots the words run over.
 struct WordAt {
   uint32_t h, tl, k, j;
 };
@@ -421,37 +431,53 @@ __device__ __forceinline__ int64_t staged_offset(const RowsArgs& a, uint32_t h0,
 // 1.5-1.8 TB/s. 400 MB of one or eight heads, head dims 80, 96, 112, 120 and 192 in bf16 and fp8:
 // 1,461-1,813 GB/s before, 5,076-6,105 now (bf16 120, eight heads kv_first 1,483 and 5,078; 112
 // combined 1,650 and 5,678); head dim 128 unchanged (5,642 and 5,613; one head 6,103 and 6,105).
-// The scatter keeps a branch around each access: its scattered stores ran 0.5-1.5 %
-// faster serialised than all in flight.
+// The scatter keeps a branch around each access, and a word past its tile moves nothing.
 template <typename T, int D, int I>
 __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_slot,
                                           const int64_t* s_head, const int64_t* s_src,
                                           int64_t layer_base, uint32_t layer, uint32_t group,
                                           int64_t t0) {
   constexpr int kThreads = threads_of(D, I);
-  constexpr int kVpt = vpt_of(D, I);
-  constexpr int kOrder = word_order(D, I);
+  constexpr int kVpt = vpt_of(D, I, sizeof(T));
   const uint32_t h0 = group * a.HG;
   const uint32_t tid = threadIdx.x;
   char* cache_w = reinterpret_cast<char*>(layer_base);
   char* rows_l = a.rows + static_cast<int64_t>(layer) * a.H * a.cap * (2 * a.half_bytes);
 
-  const bool whole = t0 + a.TS <= a.n;
-  const uint32_t slots = whole ? a.TS : static_cast<uint32_t>(a.n - t0);
-  const FastDiv div_ts = whole ? a.div_ts : a.div_ts_last;
-  // in the cache's word order the heads run inside a slot, so a last group's missing heads stay
-  // among the words (and move nothing)
-  const uint32_t heads = kOrder == 1 && h0 + a.HG > static_cast<uint32_t>(a.H) ? a.H - h0 : a.HG;
-  const uint32_t words = heads * slots * 2 * a.W;
+  // The gather's words are its tile's live ones alone, [0, words); the scatter's run over the whole
+  // tile, and those of a slot past n or a head past H move nothing.
+  const bool short_tile = D == kGather && t0 + a.TS > a.n;
+  const uint32_t slots = short_tile ? static_cast<uint32_t>(a.n - t0) : a.TS;
+  const FastDiv div_ts = short_tile ? a.div_ts_last : a.div_ts;
+  const bool few_heads = D == kGather && h0 + a.HG > static_cast<uint32_t>(a.H);
+  const uint32_t words = (few_heads ? a.H - h0 : a.HG) * slots * 2 * a.W;
 
+  // where word v lies on both sides, and whether it moves
   const auto locate = [&](uint32_t v, char*& cache, char*& staged) {
-    const WordAt at = word_at<kOrder>(a, div_ts, v);
-    const int64_t slot_off = s_slot[at.tl];
+    const WordAt at = word_at<word_order(D, I)>(a, div_ts, v);
+    const bool in_tile =
+        D == kGather || (v < words && h0 + at.h < static_cast<uint32_t>(a.H));
+    const int64_t slot_off = in_tile ? s_slot[at.tl] : -1;
     const int64_t row = I == kByPairs ? s_src[at.tl] : t0 + at.tl;
-    cache = cache_w + slot_off + s_head[at.h] + at.k * a.skv + at.j * a.sj;
+    cache = cache_w + slot_off + s_head[in_tile ? at.h : 0] + at.k * a.skv + at.j * a.sj;
     staged = rows_l + staged_offset(a, h0, row, at, sizeof(T));
-    return slot_off >= 0 && (kOrder == 1 || h0 + at.h < static_cast<uint32_t>(a.H));
+    return slot_off >= 0;
   };
+
+  // The host has checked every stride and the staging buffer for this word; the layers' bases are
+  // in device memory, so a base that does not fit it is seen here, and its rows move by bytes. A
+  // word of 16 bytes has its bases' alignment from the caller.
+  if constexpr (sizeof(T) > 1 && sizeof(T) < 16) {
+    if ((layer_base & static_cast<int64_t>(sizeof(T) - 1)) != 0) {
+      for (uint32_t v = tid; v < words; v += kThreads) {
+        char *cache, *staged;
+        if (!locate(v, cache, staged)) continue;
+        for (size_t b = 0; b < sizeof(T); b++)
+          *(D == kGather ? staged : cache)++ = *(D == kGather ? cache : staged)++;
+      }
+      return;
+    }
+  }
 
   for (uint32_t v0 = 0; v0 < words; v0 += kThreads * kVpt) {
     if (D == kGather) {
@@ -490,6 +516,11 @@ __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_sl
         }
       }
     } else {
+      // The slot scatter waits for each load before the next: its stores land in a random order,
+      // and fewer accesses in flight ran faster (65,536 permuted slots x 4 layers x 8 bf16 heads
+      // of 128: 5,764 GB/s, 5,620 with a thread's loads in flight together, 5,746 with the last
+      // load not waited for). The range and pair scatters, whose stores run along the cache, ran
+      // slower so (5,207 against 5,602 and 5,790 against 5,837), and keep their loads together.
       T w[kVpt];
       char* src[kVpt];
       char* dst[kVpt];
@@ -497,11 +528,13 @@ __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_sl
 #pragma unroll
       for (int i = 0; i < kVpt; i++) {
         const uint32_t v = v0 + i * kThreads + tid;
-        live[i] = locate(v < words ? v : words - 1, dst[i], src[i]) && v < words;
+        live[i] = locate(v, dst[i], src[i]);
       }
 #pragma unroll
-      for (int i = 0; i < kVpt; i++)
+      for (int i = 0; i < kVpt; i++) {
         if (live[i]) w[i] = load_word<T, (nt_of(D, I) & 1) != 0>(src[i]);
+        if (I == kBySlots) __builtin_amdgcn_s_waitcnt(kVmcntZero);
+      }
 #pragma unroll
       for (int i = 0; i < kVpt; i++)
         if (live[i]) store_word<T, (nt_of(D, I) & 2) != 0>(dst[i], w[i]);
@@ -586,8 +619,9 @@ struct RowsCall {
 
 template <int D, int I, typename T>
 int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const char* name) {
-  const int64_t target = I == kByPairs ? EVS_PAIRS_TILE_WORDS
-                         : D == kGather ? EVS_GATHER_TILE_WORDS : EVS_SCATTER_TILE_WORDS;
+  const int64_t target = narrow_of(sizeof(T)) *
+                         (I == kByPairs ? EVS_PAIRS_TILE_WORDS
+                         : D == kGather ? EVS_GATHER_TILE_WORDS : EVS_SCATTER_TILE_WORDS);
   const int hpt = I == kByPairs ? EVS_PAIRS_HEADS_PER_TILE
                   : D == kGather ? EVS_GATHER_HEADS_PER_TILE : EVS_SCATTER_HEADS_PER_TILE;
   a.HG = (hpt > 0 && hpt < a.H) ? hpt : a.H;
@@ -690,22 +724,34 @@ int move(const RowsCall& c, const char* name) {
   }
   a.H = static_cast<int>(c.H);
 
-  const bool vectors = c.strides[4] == 1 && aligned16(c.d * e) &&
-                       aligned16(reinterpret_cast<int64_t>(c.rows)) && aligned16(a.sb) &&
-                       aligned16(a.so) && aligned16(a.sh) && aligned16(a.skv);
-  if (vectors) {
-    a.sj = 16;
-    return launch_typed<D, I, u32x4>(a, c.L, static_cast<uint32_t>(c.d * e / 16), c.stream, name);
-  }
-  a.sj = c.strides[4] * e;
-  EVS_REQUIRE(c.d < (int64_t{1} << 24), "%s: head_dim too large", name);
-  switch (e) {
-    case 1:
-      return launch_typed<D, I, uint8_t>(a, c.L, static_cast<uint32_t>(c.d), c.stream, name);
+  // The widest word that every half-row is whole words of, on both sides; one element where a
+  // half-row's elements are not contiguous in the cache. By 8, 4 and 2 bytes instead of one
+  // element, 400 MB gathered from one combined-layout head: fp8 120 771 -> 5,560 GB/s, bf16 100
+  // 1,225 -> 5,120, fp8 100 -> 3,130, fp8 126 824 -> 3,490. The scatter: fp8 120 718 -> 5,100,
+  // bf16 100 1,134 -> 4,520.
+  int64_t word = e;
+  if (c.strides[4] == 1)
+    for (const int64_t w : {int64_t{16}, int64_t{8}, int64_t{4}, int64_t{2}}) {
+      if (w <= word) break;
+      if (((c.d * e | reinterpret_cast<int64_t>(c.rows) | a.sb | a.so | a.sh | a.skv) & (w - 1)) == 0) {
+        word = w;
+        break;
+      }
+    }
+  a.sj = c.strides[4] == 1 ? word : c.strides[4] * e;
+  EVS_REQUIRE(word == 16 || c.d < (int64_t{1} << 24), "%s: head_dim too large", name);
+  const uint32_t W = static_cast<uint32_t>(c.d * e / word);
+  switch (word) {
+    case 16:
+      return launch_typed<D, I, u32x4>(a, c.L, W, c.stream, name);
+    case 8:
+      return launch_typed<D, I, u32x2>(a, c.L, W, c.stream, name);
+    case 4:
+      return launch_typed<D, I, uint32_t>(a, c.L, W, c.stream, name);
     case 2:
-      return launch_typed<D, I, uint16_t>(a, c.L, static_cast<uint32_t>(c.d), c.stream, name);
+      return launch_typed<D, I, uint16_t>(a, c.L, W, c.stream, name);
     default:
-      return launch_typed<D, I, uint32_t>(a, c.L, static_cast<uint32_t>(c.d), c.stream, name);
+      return launch_typed<D, I, uint8_t>(a, c.L, W, c.stream, name);
   }
 }
 

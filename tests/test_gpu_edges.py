@@ -78,6 +78,42 @@ def test_passes_a_tile_does_not_fill(ext, layout, dtype, d, n):
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dtype,d", [(torch.float8_e4m3fn, 120), (torch.float8_e4m3fn, 100),
+                                     (torch.float8_e4m3fn, 126), (torch.float8_e4m3fn, 7),
+                                     (torch.bfloat16, 100), (torch.bfloat16, 126),
+                                     (torch.bfloat16, 121), (torch.float32, 6)])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_words_narrower_than_16_bytes(ext, layout, dtype, d, shift):
+    """Half-rows of whole 8-, 4-, 2- and 1-byte words, gathered and scattered, with the layers'
+    bases aligned and ``shift`` elements off (a base the word does not fit moves by bytes)."""
+    n = 37
+    layers = caches(layout, d, dtype, n_layers=L, nb=NB, h=H, seed=d)
+    slots, heads, cap, e = ragged_slots(n, d + shift), [2, 0], n + 3, layers[0].element_size()
+    st = strides_of(layers[0])
+    want = oracle.gather_rows(layers, slots, heads, cap, d, BS, st, e)
+
+    def shifted(t):  # a device copy of t whose base lies `shift` elements into its storage
+        flat = torch.empty(t.numel() + shift, dtype=t.dtype, device="cuda")
+        return flat[shift:].view(t.shape).copy_(t)
+
+    gpu = [shifted(t) for t in layers]
+    out = torch.zeros(want.nbytes, dtype=torch.uint8, device="cuda")
+    ext.gather_rows(ptrs(gpu), dev_long(slots), dev_long(heads), out.data_ptr(), cap, d, BS,
+                    list(st), e)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy().view(want.dtype).reshape(want.shape), want)
+
+    dst = caches(layout, d, dtype, n_layers=L, nb=NB, h=H, seed=d + 1)
+    gpu = [shifted(t) for t in dst]
+    oracle.scatter_rows(dst, slots, heads, want, cap, d, BS, st, e)
+    ext.scatter_rows(ptrs(gpu), dev_long(slots), dev_long(heads), out.data_ptr(), cap, d, BS,
+                     list(st), e)
+    torch.cuda.synchronize()
+    for g, w in zip(gpu, dst):
+        assert np.array_equal(bits(g), bits(w))
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("blocks", [[3], [9, 0, 77], list(range(40, 57))])
 def test_ragged_block_lists(ext, layout, blocks):
     d = 8
