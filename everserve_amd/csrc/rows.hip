@@ -12,8 +12,9 @@
 // word costs two LDS reads and no 64-bit division. Each thread then moves VPT words at a time,
 // every load in flight before the first store. A word is the widest of 16, 8, 4, 2 and 1 bytes
 // that every half-row, contiguous and aligned on both sides, is whole words of (bf16 d=128: 16
-// words of 16 bytes a half-row, fp8 d=120: 15 of 8), at least one element. Within a tile the words run along the staging buffer (K then V of one row,
-// row after row), so a wave stores whole rows: 1 KiB contiguous for bf16 d=128. For the gather
+// words of 16 bytes a half-row, fp8 d=120: 15 of 8), at least one element. Within a tile the words
+// run along the staging buffer (K then V of one row, row after row), so a wave stores whole rows:
+// 1 KiB contiguous for bf16 d=128. For the gather
 // the tile numbers run through a slot range's head groups first, so the workgroups reading the
 // heads of one cache block (adjacent in every paged layout) are neighbours, dealt round-robin to
 // the XCDs; the slot and pair scatters' XCD remap (xcd_tile) keeps runs of 64 neighbouring tiles
@@ -27,6 +28,8 @@
 // workgroup but slows these kernels, whose index prologue needs every resident workgroup to hide
 // its latency; each wave reading its own rows' ids with scalar loads, no LDS and no barrier
 // (2 % slower: the per-lane choice among the wave's rows costs more than the barrier).
+
+#include <numeric>
 
 #include "common.hpp"
 
@@ -172,8 +175,16 @@ enum Dir : int { kGather = 0, kScatter = 1 };
 // range k with first_rows[k] <= t < first_rows[k + 1].
 enum Index : int { kBySlots = 0, kByBlocks = 1, kByPairs = 2, kByRanges = 3 };
 
-constexpr int threads_of(int d, int i) {
-  return i == kByPairs ? EVS_PAIRS_THREADS : d == kGather ? EVS_GATHER_THREADS : EVS_SCATTER_THREADS;
+// A kernel's form. kSpanning (slot and range scatters): the tile spans heads, see launch_typed.
+// kSmall (the gather of 16-byte words): half the threads and half the tile.
+enum Form : int { kPlain = 0, kSpanning = 1, kSmall = 2 };
+
+constexpr int threads_of(int d, int i, int form = kPlain) {
+  return i == kByPairs        ? EVS_PAIRS_THREADS
+         : form == kSmall     ? EVS_GATHER_THREADS / 2
+         : d == kGather       ? EVS_GATHER_THREADS
+         : form == kSpanning  ? 256
+                              : EVS_SCATTER_THREADS;
 }
 // A narrower word's passes and tiles hold more of them: 2x at 8 bytes (the same bytes a tile), 4x
 // below, where the work is the address arithmetic a word takes. 400 MB gathered from one head, 4x
@@ -191,8 +202,12 @@ constexpr int nt_of(int d, int i) {
                            : EVS_SCATTER_NT;
 }
 // the gather's words run along the staging buffer, so that its tile's words are all live ones
-constexpr int order_of(int d) { return d == kGather ? 1 : EVS_SCATTER_ORDER; }
-constexpr int word_order(int d, int i) { return i == kByPairs ? EVS_PAIRS_ORDER : order_of(d); }
+constexpr int word_order(int d, int i, int form) {
+  return i == kByPairs       ? EVS_PAIRS_ORDER
+         : d == kGather      ? 1
+         : form == kSpanning ? 2
+                             : EVS_SCATTER_ORDER;
+}
 static_assert(threads_of(kGather, kBySlots) >= kMaxTileSlots &&
                   threads_of(kScatter, kBySlots) >= kMaxTileSlots &&
                   threads_of(kScatter, kByPairs) >= kMaxTileSlots,
@@ -405,6 +420,10 @@ __device__ __forceinline__ WordAt word_at(const RowsArgs& a, const FastDiv& div_
     // v = ((k * TS + tl) * HG + h) * W + j
     a.div_h.divmod(q, q2, w.h);
     div_ts.divmod(q2, w.k, w.tl);
+  } else if (kOrder == 2) {
+    // v = ((tl * HG + h) * 2 + k) * W + j: the heads' rows of one slot, slot after slot
+    w.k = q & 1u;
+    a.div_h.divmod(q >> 1, w.tl, w.h);
   } else {
     // v = ((h * TS + tl) * 2 + k) * W + j: K then V of one staged row, row after row
     w.k = q & 1u;
@@ -420,6 +439,45 @@ __device__ __forceinline__ int64_t staged_offset(const RowsArgs& a, uint32_t h0,
          w.k * a.half_bytes + static_cast<int64_t>(w.j) * word_bytes;
 }
 
+// Move kWords words a thread of a gather's tile, kThreads words apart from word v0 + its number
+// on, every load in flight before the first store. The last of the wave's kWords runs of 64 may
+// end past the tile's words.
+template <int kWords, typename T, int kThreads, int kNt, typename Locate>
+__device__ __forceinline__ void gather_words(uint32_t v0, uint32_t words, const Locate& locate) {
+  T w[kWords];
+  char* src[kWords];
+  char* dst[kWords];
+#pragma unroll
+  for (int i = 0; i < kWords; i++) {
+    const uint32_t at = v0 + i * kThreads + threadIdx.x;
+    locate(i == kWords - 1 && at >= words ? words - 1 : at, src[i], dst[i]);
+  }
+  // Each load stays where it is issued (the scheduler otherwise issued the second word's
+  // load first, after the first's address work, so the first store waited for both loads):
+  // now the first word's store waits for its own load only. 9-11 interleaved rounds on two
+  // boxes: C2 6,110-6,113 against 6,096-6,098 GB/s, C3 6,159 against 6,124, one bf16 head
+  // 6,266 against 6,197, the combined layout 6,090 against 6,057, blocks_first unchanged.
+#pragma unroll
+  for (int i = 0; i < kWords; i++) {
+    w[i] = load_word<T, (kNt & 1) != 0>(src[i]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < kWords; i++)
+    store_word<T, (kNt & 2) != 0, EVS_GATHER_STORE_SC1 != 0>(dst[i], w[i]);
+}
+
+// A wave's words of the tile from v0 on (`wave`: its first thread's number): kWords a thread for as
+// long as the tile has them, then by halves.
+template <int kWords, typename T, int kThreads, int kNt, typename Locate>
+__device__ __forceinline__ void gather_by_halves(uint32_t v0, uint32_t wave, uint32_t words,
+                                                 const Locate& locate) {
+  for (; v0 + wave + (kWords - 1) * kThreads < words; v0 += kWords * kThreads)
+    gather_words<kWords, T, kThreads, kNt>(v0, words, locate);
+  if constexpr (kWords > 1)
+    gather_by_halves<kWords / 2, T, kThreads, kNt>(v0, wave, words, locate);
+}
+
 // Move one tile's words: the slots' offsets and the heads' are in LDS, and for the pair scatter
 // the staged rows'. A wave past the tile's last word leaves; in the wave that holds the last word
 // the gather's lanes past it move that word again, which costs nothing (the same lines in the
@@ -432,12 +490,12 @@ __device__ __forceinline__ int64_t staged_offset(const RowsArgs& a, uint32_t h0,
 // 1,461-1,813 GB/s before, 5,076-6,105 now (bf16 120, eight heads kv_first 1,483 and 5,078; 112
 // combined 1,650 and 5,678); head dim 128 unchanged (5,642 and 5,613; one head 6,103 and 6,105).
 // The scatter keeps a branch around each access, and a word past its tile moves nothing.
-template <typename T, int D, int I>
+template <typename T, int D, int I, int F>
 __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_slot,
                                           const int64_t* s_head, const int64_t* s_src,
                                           int64_t layer_base, uint32_t layer, uint32_t group,
                                           int64_t t0) {
-  constexpr int kThreads = threads_of(D, I);
+  constexpr int kThreads = threads_of(D, I, F);
   constexpr int kVpt = vpt_of(D, I, sizeof(T));
   const uint32_t h0 = group * a.HG;
   const uint32_t tid = threadIdx.x;
@@ -454,7 +512,7 @@ __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_sl
 
   // where word v lies on both sides, and whether it moves
   const auto locate = [&](uint32_t v, char*& cache, char*& staged) {
-    const WordAt at = word_at<word_order(D, I)>(a, div_ts, v);
+    const WordAt at = word_at<word_order(D, I, F)>(a, div_ts, v);
     const bool in_tile =
         D == kGather || (v < words && h0 + at.h < static_cast<uint32_t>(a.H));
     const int64_t slot_off = in_tile ? s_slot[at.tl] : -1;
@@ -479,73 +537,55 @@ __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_sl
     }
   }
 
-  for (uint32_t v0 = 0; v0 < words; v0 += kThreads * kVpt) {
-    if (D == kGather) {
-      const uint32_t wave = v0 + __builtin_amdgcn_readfirstlane(tid & ~63u);
-      if (wave >= words) break;  // this wave's later passes lie further on still
-      if (wave + (kVpt - 1) * kThreads < words) {
-        T w[kVpt];
-        char* src[kVpt];
-        char* dst[kVpt];
-#pragma unroll
-        for (int i = 0; i < kVpt; i++) {
-          const uint32_t v = v0 + i * kThreads + tid;
-          locate(i == kVpt - 1 && v >= words ? words - 1 : v, src[i], dst[i]);
-        }
-        // Each load stays where it is issued (the scheduler otherwise issued the second word's
-        // load first, after the first's address work, so the first store waited for both loads):
-        // now the first word's store waits for its own load only. 9-11 interleaved rounds on two
-        // boxes: C2 6,110-6,113 against 6,096-6,098 GB/s, C3 6,159 against 6,124, one bf16 head
-        // 6,266 against 6,197, the combined layout 6,090 against 6,057, blocks_first unchanged.
-#pragma unroll
-        for (int i = 0; i < kVpt; i++) {
-          w[i] = load_word<T, (nt_of(D, I) & 1) != 0>(src[i]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int i = 0; i < kVpt; i++)
-          store_word<T, (nt_of(D, I) & 2) != 0, EVS_GATHER_STORE_SC1 != 0>(dst[i], w[i]);
-      } else {
-        // a pass that the tile does not fill: its words one at a time
-        for (uint32_t v1 = v0; v1 + (wave - v0) < words; v1 += kThreads) {
-          const uint32_t v = v1 + tid;
-          char *src, *dst;
-          locate(v < words ? v : words - 1, src, dst);
-          store_word<T, (nt_of(D, I) & 2) != 0, EVS_GATHER_STORE_SC1 != 0>(
-              dst, load_word<T, (nt_of(D, I) & 1) != 0>(src));
-        }
-      }
+  if constexpr (D == kGather) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid & ~63u);
+    if constexpr (kVpt > 2) {
+      gather_by_halves<kVpt, T, kThreads, nt_of(D, I)>(0, wave, words, locate);
     } else {
-      // The slot scatter waits for each load before the next: its stores land in a random order,
-      // and fewer accesses in flight ran faster (65,536 permuted slots x 4 layers x 8 bf16 heads
-      // of 128: 5,764 GB/s, 5,620 with a thread's loads in flight together, 5,746 with the last
-      // load not waited for). The range and pair scatters, whose stores run along the cache, ran
-      // slower so (5,207 against 5,602 and 5,790 against 5,837), and keep their loads together.
-      T w[kVpt];
-      char* src[kVpt];
-      char* dst[kVpt];
-      bool live[kVpt];
-#pragma unroll
-      for (int i = 0; i < kVpt; i++) {
-        const uint32_t v = v0 + i * kThreads + tid;
-        live[i] = locate(v, dst[i], src[i]);
+      // the same for two words a thread, written out: this form ran 0.3-0.8 % faster for them
+      for (uint32_t v0 = 0; v0 < words; v0 += kThreads * kVpt) {
+        if (v0 + wave >= words) break;  // this wave's later passes lie further on still
+        if (v0 + wave + (kVpt - 1) * kThreads < words) {
+          gather_words<kVpt, T, kThreads, nt_of(D, I)>(v0, words, locate);
+        } else {
+          for (uint32_t v1 = v0; v1 + wave < words; v1 += kThreads)
+            gather_words<1, T, kThreads, nt_of(D, I)>(v1, words, locate);
+        }
       }
-#pragma unroll
-      for (int i = 0; i < kVpt; i++) {
-        if (live[i]) w[i] = load_word<T, (nt_of(D, I) & 1) != 0>(src[i]);
-        if (I == kBySlots) __builtin_amdgcn_s_waitcnt(kVmcntZero);
-      }
-#pragma unroll
-      for (int i = 0; i < kVpt; i++)
-        if (live[i]) store_word<T, (nt_of(D, I) & 2) != 0>(dst[i], w[i]);
     }
+    return;
+  }
+  for (uint32_t v0 = 0; v0 < words; v0 += kThreads * kVpt) {
+    // The slot scatter waits for each load before the next: its stores land in a random order,
+    // and fewer accesses in flight ran faster (65,536 permuted slots x 4 layers x 8 bf16 heads
+    // of 128: 5,764 GB/s, 5,620 with a thread's loads in flight together, 5,746 with the last
+    // load not waited for). The range and pair scatters, whose stores run along the cache, ran
+    // slower so (5,207 against 5,602 and 5,790 against 5,837), and keep their loads together, as
+    // does the slot scatter that spans heads (bf16 112, 8 heads: 5,235 against 4,908).
+    T w[kVpt];
+    char* src[kVpt];
+    char* dst[kVpt];
+    bool live[kVpt];
+#pragma unroll
+    for (int i = 0; i < kVpt; i++) {
+      const uint32_t v = v0 + i * kThreads + tid;
+      live[i] = locate(v, dst[i], src[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < kVpt; i++) {
+      if (live[i]) w[i] = load_word<T, (nt_of(D, I) & 1) != 0>(src[i]);
+      if (I == kBySlots && F == kPlain) __builtin_amdgcn_s_waitcnt(kVmcntZero);
+    }
+#pragma unroll
+    for (int i = 0; i < kVpt; i++)
+      if (live[i]) store_word<T, (nt_of(D, I) & 2) != 0>(dst[i], w[i]);
   }
 }
 
 // Fill a tile's slot and head offsets into LDS. The first wave reads both index entries before it
 // uses either, so that the two reads are in flight together; its lanes past the tile's slots and
 // heads read the tile's last entry again, so that the reads touch only the tile's own lines.
-template <int D, int I>
+template <int D, int I, int F>
 __device__ __forceinline__ void tile_offsets(const RowsArgs& a, const TileId& id, int64_t t0,
                                              int64_t* s_slot, int64_t* s_head, int64_t* s_src) {
   const int tid = threadIdx.x;
@@ -573,13 +613,13 @@ __device__ __forceinline__ void tile_offsets(const RowsArgs& a, const TileId& id
     }
     if (tid < a.HG && h0 + tid < a.H) s_head[tid] = head * a.sh;
   }
-  for (int h = kMaxTileSlots + tid; h < a.HG && h0 + h < a.H; h += threads_of(D, I))
+  for (int h = kMaxTileSlots + tid; h < a.HG && h0 + h < a.H; h += threads_of(D, I, F))
     s_head[h] = a.heads[h0 + h] * a.sh;
 }
 
 // One tile per workgroup.
-template <typename T, int D, int I>
-__global__ __launch_bounds__(threads_of(D, I)) void move_rows(RowsArgs a) {
+template <typename T, int D, int I, int F>
+__global__ __launch_bounds__(threads_of(D, I, F)) void move_rows(RowsArgs a) {
   __shared__ int64_t s_slot[kMaxTileSlots];  // byte offset of a slot's row in a layer, -1: none
   __shared__ int64_t s_head[kMaxHeads];      // byte offset of a head slot in a row group
   __shared__ int64_t s_src[I == kByPairs ? kMaxTileSlots : 1];  // kByPairs: staged row of a slot
@@ -590,9 +630,9 @@ __global__ __launch_bounds__(threads_of(D, I)) void move_rows(RowsArgs a) {
   // keep this uniform read scalar (the store might alias it), and a vector read of it made every
   // pass wait for all memory operations in flight (measured 8 % slower).
   const int64_t layer_base = a.layer_ptrs[id.layer];
-  tile_offsets<D, I>(a, id, t0, s_slot, s_head, s_src);
+  tile_offsets<D, I, F>(a, id, t0, s_slot, s_head, s_src);
   __syncthreads();
-  move_tile<T, D, I>(a, s_slot, s_head, s_src, layer_base, id.layer, id.group, t0);
+  move_tile<T, D, I, F>(a, s_slot, s_head, s_src, layer_base, id.layer, id.group, t0);
 }
 
 struct RowsCall {
@@ -617,14 +657,22 @@ struct RowsCall {
   int64_t nranges = 0;                  // kByRanges
 };
 
-template <int D, int I, typename T>
-int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const char* name) {
-  const int64_t target = narrow_of(sizeof(T)) *
-                         (I == kByPairs ? EVS_PAIRS_TILE_WORDS
-                         : D == kGather ? EVS_GATHER_TILE_WORDS : EVS_SCATTER_TILE_WORDS);
-  const int hpt = I == kByPairs ? EVS_PAIRS_HEADS_PER_TILE
-                  : D == kGather ? EVS_GATHER_HEADS_PER_TILE : EVS_SCATTER_HEADS_PER_TILE;
-  a.HG = (hpt > 0 && hpt < a.H) ? hpt : a.H;
+// Half-rows that are no whole number of 128-byte memory lines leave lines that two heads' or two
+// tiles' words share. Two workgroups that each write a part of a line, or read it, on different
+// XCDs move it twice, so the tile's heads and slots are chosen to cover lines whole.
+constexpr int64_t kLine = 128;
+
+// The fewest runs of `bytes`, one after another, that fill whole lines.
+int64_t per_line(int64_t bytes) { return kLine / std::gcd(kLine, bytes); }
+
+// Launch tiles of `hg` heads (0: all) and about `target` words. lines: a gather's tile may be cut
+// or grown to whole lines of its rows.
+template <int D, int I, int F, typename T>
+int launch_tiles(RowsArgs a, int64_t L, int64_t hg, int64_t target, hipStream_t stream,
+                 const char* name, bool lines = true) {
+  const uint32_t W = a.W;
+  const int64_t threads = threads_of(D, I, F);
+  a.HG = static_cast<int>(hg > 0 && hg < a.H ? hg : a.H);
   a.group_fastest = D == kGather      ? EVS_GATHER_GROUP_FASTEST
                     : I == kByRanges ? EVS_RANGES_GROUP_FASTEST
                                      : EVS_SCATTER_GROUP_FASTEST;
@@ -632,31 +680,127 @@ int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const ch
                 : I == kByRanges ? EVS_RANGES_XCD_CHUNK
                 : D == kGather ? EVS_GATHER_XCD_CHUNK : EVS_SCATTER_XCD_CHUNK;
   const int64_t groups = (a.H + a.HG - 1) / a.HG;
-  if (D == kGather && I != kByPairs && groups == 1) a.xcd_chunk = EVS_GATHER_XCD_CHUNK_ONE_GROUP;
+  if (D == kGather && groups == 1) a.xcd_chunk = EVS_GATHER_XCD_CHUNK_ONE_GROUP;
   const int64_t per_slot = static_cast<int64_t>(a.HG) * 2 * W;
   int64_t ts = target / per_slot;
+  if (D == kGather && lines) {
+    // Whole lines of each head's staged rows, where that leaves no more than an eighth of the
+    // tile's words empty or needs no more than two tiles' words (of 8 or 16 bytes). 400 MB of one
+    // head: bf16 120 (16 slots a tile for 17) 5,971 against 5,148 GB/s, fp8 80 (48 for 51) 5,967
+    // against 5,142; bf16 100 (20 to 16) would run at 5,139 against 5,465, bf16 126 (8 to 16, two
+    // heads, 4-byte words) at 4,865 against 5,361.
+    const int64_t whole = per_line(2 * a.half_bytes);
+    if (ts / whole * whole * 8 >= ts * 7)
+      ts = ts / whole * whole;
+    else if (sizeof(T) >= 8 && ts < whole && whole * per_slot <= 2 * target)
+      ts = whole;
+  }
   ts = ts < 1 ? 1 : (ts > kMaxTileSlots ? kMaxTileSlots : ts);
   if (ts > a.n) ts = a.n;
   const int64_t tiles = (a.n + ts - 1) / ts;
   const int64_t grid = tiles * groups * L;
   EVS_REQUIRE(ts * per_slot < (int64_t{1} << 31), "%s: a tile of %lld words is too large", name,
               static_cast<long long>(ts * per_slot));
-  // HIP on AMD GPUs takes at most 2^32 - 1 work-items along x (gridDim.x * blockDim.x)
-  EVS_REQUIRE(grid * threads_of(D, I) < (int64_t{1} << 32),
+  // HIP on AMD GPUs takes at most 2^32 - 1 work-items along x (gridDim.x * blockDim.x). A shape
+  // chosen for its lines may leave some of a tile's words empty, and so need more workgroups: a
+  // call that is too large for it still fits the plain one.
+  if (I != kByPairs && lines && grid * threads >= (int64_t{1} << 32))
+    return launch_tiles<D, I, kPlain, T>(
+        a, L, D == kGather ? EVS_GATHER_HEADS_PER_TILE : EVS_SCATTER_HEADS_PER_TILE,
+        (D == kGather ? EVS_GATHER_TILE_WORDS : EVS_SCATTER_TILE_WORDS) * narrow_of(sizeof(T)),
+        stream, name, false);
+  EVS_REQUIRE(grid * threads < (int64_t{1} << 32),
               "%s: %lld workgroups of %d threads exceed the launch limit of 2^32 - 1 work-items; "
-              "split the call by layers", name, static_cast<long long>(grid), threads_of(D, I));
+              "split the call by layers", name, static_cast<long long>(grid),
+              static_cast<int>(threads));
   a.TS = static_cast<int>(ts);
-  a.W = W;
   a.div_w = FastDiv(W);
   a.div_h = FastDiv(static_cast<uint32_t>(a.HG));
   a.div_ts = FastDiv(static_cast<uint32_t>(ts));
   a.div_ts_last = FastDiv(static_cast<uint32_t>(a.n - (tiles - 1) * ts));
   a.div_tiles = FastDiv(static_cast<uint32_t>(tiles));
   a.div_groups = FastDiv(static_cast<uint32_t>(groups));
-  hipLaunchKernelGGL((move_rows<T, D, I>), dim3(static_cast<uint32_t>(grid)),
-                     dim3(threads_of(D, I)), 0, stream, a);
+  hipLaunchKernelGGL((move_rows<T, D, I, F>), dim3(static_cast<uint32_t>(grid)),
+                     dim3(static_cast<uint32_t>(threads)), 0, stream, a);
   EVS_LAUNCHED(name);
   return EVS_OK;
+}
+
+// Heads of a gather's tile. Two, or four where the heads of a slot lie side by side in half-rows of
+// at most 256 bytes (four slots a tile or more) and the rows of two neighbouring heads in the
+// staging buffer are at most 4 MiB apart: a tile writes all its heads at once, and heads 8 MiB
+// apart and more meet on the same memory channels. bf16, 8 heads of 128,
+// 32 layers, four against two: 8,192 slots (4 MiB) 6,310 against 6,088 GB/s, 5,001 6,303 against
+// 6,014, 1,000 6,035 against 5,919; 16,384 slots (8 MiB) 6,111 against 6,160, 65,536 (8 layers)
+// 5,915 against 5,980; four heads in all, 8,192 slots 5,956 against 6,213. Where the half-rows are no whole lines: as many heads as fill them, or all,
+// if two tiles' words hold whole lines of those heads' staged rows. 400 MB, 8 heads: bf16 80 (4
+// heads) 5,541 against 5,124 with two, fp8 112 (8) 5,341 against 4,445, fp8 120 (8) 4,957 against
+// 3,517; bf16 100, whose 8 heads do not fit, 5,072 with four against 3,865 with 8.
+int64_t gather_heads(const RowsArgs& a, int64_t target) {
+  if (a.sh != a.half_bytes) return EVS_GATHER_HEADS_PER_TILE;
+  const int64_t whole = per_line(a.half_bytes);
+  const int64_t hg = whole < a.H ? whole : a.H;
+  if (whole > 2 && whole <= 16 && a.H % hg == 0 &&
+      per_line(2 * a.half_bytes) * hg * 2 * a.W <= 2 * target)
+    return hg;
+  return a.H > 4 && a.H % 4 == 0 && a.half_bytes <= 256 &&
+                 a.cap * 2 * a.half_bytes <= (int64_t{4} << 20)
+             ? 4
+             : EVS_GATHER_HEADS_PER_TILE;
+}
+
+// Heads of a spanning scatter's tile: enough to fill whole lines of a slot's heads (or all of
+// them), the most of those that leave the fewest of a pass's words without work.
+int64_t span_heads(const RowsArgs& a, int64_t target) {
+  const int64_t H = a.H, whole = per_line(a.half_bytes), head_words = 2 * a.W;
+  int64_t best = whole < H ? whole : H, best_live = 0;
+  for (int64_t hg = whole; hg < H + whole; hg += whole) {
+    const int64_t h = hg < H ? hg : H;
+    const int64_t slots = target / (h * head_words);
+    if (slots == 0) break;
+    const int64_t groups = (H + h - 1) / h;
+    const int64_t live = H * slots * head_words * 256 / (groups * target);  // of 256
+    if (live >= best_live) {
+      best = h;
+      best_live = live;
+    }
+  }
+  return best;
+}
+
+template <int D, int I, typename T>
+int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const char* name) {
+  a.W = W;
+  constexpr int64_t kNarrow = narrow_of(sizeof(T));
+  if constexpr (I == kByPairs) {
+    return launch_tiles<D, I, kPlain, T>(a, L, EVS_PAIRS_HEADS_PER_TILE,
+                                        EVS_PAIRS_TILE_WORDS * kNarrow, stream, name);
+  } else if constexpr (D == kGather) {
+    constexpr int64_t target = EVS_GATHER_TILE_WORDS * kNarrow;
+    const int64_t hg = gather_heads(a, target);
+    if constexpr (sizeof(T) == 16) {
+      // Two heads a tile of several (their rows far apart, see gather_heads), in whole lines: half
+      // the tile. bf16 heads of 128, 32 layers, 8 heads: 16,384 slots 6,179 against 6,168 GB/s,
+      // 32,768 5,986 against 5,912; 4 heads of 64, 32,768 6,183 against 6,157. Four heads a tile,
+      // one head and the combined layout gained nothing from it.
+      if (hg == 2 && a.H > 2 && a.sh == a.half_bytes && per_line(a.half_bytes) == 1)
+        return launch_tiles<D, I, kSmall, T>(a, L, hg, target / 2, stream, name);
+    }
+    return launch_tiles<D, I, kPlain, T>(a, L, hg, target, stream, name);
+  } else {
+    // Where a slot's heads lie side by side in half-rows that are no whole lines, the scatter of
+    // one head a tile writes each line in parts from several workgroups: the tile spans heads
+    // instead, one slot's heads after another. 400 MB, 8 heads, by slots: fp8 64 4,519 -> 5,630
+    // GB/s, 96 2,220 -> 5,290, 120 1,910 -> 4,627, bf16 80 2,950 -> 5,358, 112 3,498 -> 5,235, 120
+    // 3,104 -> 5,347; by 1,034 ranges: fp8 64 3,823 -> 5,423, bf16 80 2,834 -> 4,921. Half-rows of
+    // whole lines run faster one head a tile (bf16 128: 5,862 against 5,627 spanning).
+    if (a.H > 1 && a.sh == a.half_bytes && per_line(a.half_bytes) > 1) {
+      constexpr int64_t target = 512 * kNarrow;  // one pass of the 256 threads
+      return launch_tiles<D, I, kSpanning, T>(a, L, span_heads(a, target), target, stream, name);
+    }
+    return launch_tiles<D, I, kPlain, T>(a, L, EVS_SCATTER_HEADS_PER_TILE,
+                                        EVS_SCATTER_TILE_WORDS * kNarrow, stream, name);
+  }
 }
 
 // The checks of a call's arguments. *moves is false when the call has nothing to move (no slot,

@@ -114,6 +114,45 @@ def test_words_narrower_than_16_bytes(ext, layout, dtype, d, shift):
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("heads_total", [2, 5, 8, 12])
+@pytest.mark.parametrize("dtype,d", [(torch.float8_e4m3fn, 64), (torch.float8_e4m3fn, 96),
+                                     (torch.float8_e4m3fn, 120), (torch.bfloat16, 80),
+                                     (torch.bfloat16, 112), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("n", [3, 41])
+def test_head_groups_of_every_tile_shape(ext, layout, heads_total, dtype, d, n):
+    """Head counts the tiles' head groups divide and do not, held in another order than the
+    cache's, with half-rows of whole memory lines and not: the gather, the slot scatter and the
+    range scatter (which span heads where the lines are shared)."""
+    layers = caches(layout, d, dtype, n_layers=L, nb=NB, h=heads_total, seed=d + n)
+    rng = np.random.default_rng(heads_total)
+    slots, heads = ragged_slots(n, d), rng.permutation(heads_total).tolist()
+    cap, e, st = n + 3, layers[0].element_size(), strides_of(layers[0])
+    want = oracle.gather_rows(layers, slots, heads, cap, d, BS, st, e)
+    gpu = [t.cuda() for t in layers]
+    out = torch.zeros(want.nbytes, dtype=torch.uint8, device="cuda")
+    ext.gather_rows(ptrs(gpu), dev_long(slots), dev_long(heads), out.data_ptr(), cap, d, BS,
+                    list(st), e)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy().view(want.dtype).reshape(want.shape), want)
+
+    starts = np.arange(0, 5 * n, 5)  # n ranges of one slot, 4 apart, as a restore's ascend
+    first = np.arange(n + 1)
+    for slot_list, by_ranges in ((slots, False), (starts.tolist(), True)):
+        dst = caches(layout, d, dtype, n_layers=L, nb=NB, h=heads_total, seed=d + n + 1)
+        gpu = [t.cuda() for t in dst]
+        oracle.scatter_rows(dst, slot_list, heads, want, cap, d, BS, st, e)
+        if by_ranges:
+            ext.scatter_ranges(ptrs(gpu), dev_long(starts), dev_long(first), n, dev_long(heads),
+                               out.data_ptr(), cap, d, BS, list(st), e)
+        else:
+            ext.scatter_rows(ptrs(gpu), dev_long(slots), dev_long(heads), out.data_ptr(), cap, d,
+                             BS, list(st), e)
+        torch.cuda.synchronize()
+        for g, w in zip(gpu, dst):
+            assert np.array_equal(bits(g), bits(w))
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("blocks", [[3], [9, 0, 77], list(range(40, 57))])
 def test_ragged_block_lists(ext, layout, blocks):
     d = 8
