@@ -144,22 +144,21 @@ int evs_scatter_ranges(const int64_t* layer_ptrs, int64_t num_layers, const int6
  * slot id (padding) lands wherever its low bits put it, and evs_scatter_pairs skips it.
  * `workspace` is device memory of at least evs_order_pairs_workspace(num_pairs, key_bits) bytes,
  * 256-byte aligned, owned by the caller; the call allocates nothing and does not synchronise.
- * The sort clears its own counters in the workspace with hipMemsetAsync, so keep this call out
- * of captured HIP graphs. num_pairs < 2^31. No counterpart in the reference: it orders the restore's writes (see
+ * Above 2^20 pairs the sort clears its own counters in the workspace with hipMemsetAsync, so keep
+ * this call out of captured HIP graphs. num_pairs < 2^31. No counterpart in the reference: it orders the restore's writes (see
  * evs_scatter_pairs); the host-side equivalent is everserve_amd.state.restore.destination_order. */
 int evs_order_pairs_workspace(int64_t num_pairs, int key_bits, int64_t* bytes);
 int evs_order_pairs(const int64_t* slots, int64_t num_pairs, int key_bits, int64_t* slots_out,
                     int64_t* rows_out, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* evs_order_pairs without a workspace argument, for callers that cannot allocate device memory
- * (tight serving loops, harnesses that forbid hipMalloc). Not for HIP graph capture: see the
- * memset below. No counterpart in the reference. Its scratch is a file-scope device array of
+ * (tight serving loops, harnesses that forbid hipMalloc). Not for HIP graph capture: every call
+ * on a GPU shares its scratch. No counterpart in the reference. Its scratch is a file-scope device array of
  * EVS_ORDER_STATIC_SCRATCH_BYTES that every GPU the library runs on holds until the process ends;
  * num_pairs is at most EVS_ORDER_STATIC_MAX_PAIRS (a larger call is refused with a message, and
  * nothing is enqueued). Calls on one GPU share that GPU's array: two calls that overlap on one GPU
  * (on different streams, or from different threads) race and give wrong results, so order them.
- * The call allocates nothing and does not synchronise; like evs_order_pairs, rocPRIM clears its
- * counters with hipMemsetAsync, so keep it out of captured graphs. */
+ * The call allocates nothing and does not synchronise. */
 #define EVS_ORDER_STATIC_MAX_PAIRS (1 << 20)
 #define EVS_ORDER_STATIC_SCRATCH_BYTES (32 << 20)
 int evs_order_pairs_static(const int64_t* slots, int64_t num_pairs, int key_bits,

@@ -36,6 +36,41 @@ def test_the_device_order_is_the_host_order(ext, n, num_slots):
     assert np.array_equal(got_s[keep], want_s) and np.array_equal(got_r[keep], want_r)
 
 
+# one workgroup's sort and its halves (2,048 and 8,192 pairs), tiles of 2,048 and of 4,096 (past
+# 2^19 pairs), and the size past which rocPRIM's sort takes over
+EDGES = [63, 2048, 2049, 8192, 8193, 20_481, (1 << 19) + 1, 1 << 20, (1 << 20) + 1]
+
+
+@pytest.mark.parametrize("n", EDGES)
+@pytest.mark.parametrize("bits", [5, 18, 30, 64])
+def test_every_size_and_width_is_a_stable_sort_of_the_low_bits(ext, n, bits):
+    """Ids with bits above the compared ones, many ties and negative ids, at the edges of the
+    sort's tiles and dispatch, against numpy's stable sort of the low bits as unsigned."""
+    rng = np.random.default_rng(n + bits)
+    slots = rng.integers(-(1 << 40), 1 << 40, n) if bits == 64 else rng.integers(0, 1 << 20, n)
+    slots[rng.random(n) < 0.05] = -1
+    low = slots.astype(np.uint64) & np.uint64((1 << bits) - 1)
+    want = np.argsort(low, kind="stable")
+    got_s, got_r = on_device(ext, slots, 1 << bits)
+    assert np.array_equal(got_r, want)
+    assert np.array_equal(got_s, slots[want])
+
+
+@pytest.mark.parametrize("n", [2048, 8193])
+@pytest.mark.parametrize("bits", [8, 18, 20])
+def test_the_ids_sorted_where_they_lie(ext, n, bits):
+    """slots_out is the slot list itself: one to three passes, none of which may write ids that
+    another workgroup has still to read."""
+    slots = np.random.default_rng(n).integers(0, 1 << bits, n)
+    dev = torch.from_numpy(slots.copy()).cuda()
+    rows = torch.empty_like(dev)
+    ext.order_pairs(dev, 1 << bits, out=(dev, rows))
+    torch.cuda.synchronize()
+    want = np.argsort(slots, kind="stable")
+    assert np.array_equal(rows.cpu().numpy(), want)
+    assert np.array_equal(dev.cpu().numpy(), slots[want])
+
+
 def test_ties_keep_their_listed_order(ext):
     slots = np.array([7, 3, 7, 3, 0, 7], dtype=np.int64)
     got_s, got_r = on_device(ext, slots, 8)
