@@ -23,6 +23,7 @@ torch's current stream of the tensors' device, as the reference's ``gather_rows`
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import functools
 import json
@@ -267,25 +268,52 @@ def open_library(path: Path | None = None) -> ctypes.CDLL:
     return lib
 
 
+# A small call costs the host more than the GPU, and these helpers were most of it: through
+# torch.cuda.current_stream, torch.cuda.device and sets of torch.device objects a gather of 8 slots
+# took 8.4 us of host time and order_pairs 13.2, through the raw stream and the devices' numbers
+# 6.2 and 6.3, of which HIP's launch is 3.2.
+_FIVE = ctypes.c_int64 * 5
+_HERE = contextlib.nullcontext()
+
+
 def _stream_of(device) -> int:
+    """The handle of torch's current stream of ``device``."""
     import torch
 
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
+
+
+def _on_device_of(t):
+    """A context in which ``t``'s GPU is the current device: nothing to do when it is already."""
+    import torch
+
+    return _HERE if torch._C._cuda_getDevice() == t.get_device() else torch.cuda.device(t.device)
 
 
 def _device_ptr(t, what: str, dtype) -> int:
     """A device tensor's address, after checking it is on the GPU and of ``dtype``."""
+    if t.is_cuda and t.dtype == dtype and t.is_contiguous():
+        return t.data_ptr()
     if not t.is_cuda:
         raise RuntimeError(f"{what} must be on the device")
     if t.dtype != dtype:
         raise RuntimeError(f"{what} must be {dtype}, got {t.dtype}")
-    if not t.is_contiguous():
-        raise RuntimeError(f"{what} must be contiguous")
-    return t.data_ptr()
+    raise RuntimeError(f"{what} must be contiguous")
 
 
 def _one_device(what: str, *tensors) -> None:
     """The tensors a launch reads must all be on one GPU: the kernel runs there."""
+    at = None
+    for t in tensors:
+        if t is not None:
+            if at is None:
+                at = t.get_device()
+            elif t.get_device() != at:
+                break
+    else:
+        return
     devices = {t.device for t in tensors if t is not None}
     if len(devices) > 1:
         raise RuntimeError(f"{what}: tensors on several devices ({sorted(map(str, devices))})")
@@ -337,8 +365,8 @@ class Kernels:
         sp = _device_ptr(slots, "gather_rows: slots", torch.long)
         hp = _device_ptr(heads, "gather_rows: heads", torch.long)
         _one_device("gather_rows", layer_ptrs, slots, heads)
-        st = (ctypes.c_int64 * 5)(*[int(s) for s in strides])
-        with torch.cuda.device(slots.device):
+        st = _FIVE(*[int(s) for s in strides])
+        with _on_device_of(slots):
             self._check(
                 self._lib.evs_gather_rows(
                     lp, layer_ptrs.numel(), sp, slots.numel(), hp, heads.numel(), int(out_ptr),
@@ -395,8 +423,8 @@ class Kernels:
             if slots_out.numel() < block_ids.numel() * block_size:
                 raise RuntimeError("gather_blocks: slots_out holds fewer than blocks * block_size")
         _one_device("gather_blocks", layer_ptrs, block_ids, heads, slots_out)
-        st = (ctypes.c_int64 * 5)(*[int(s) for s in strides])
-        with torch.cuda.device(block_ids.device):
+        st = _FIVE(*[int(s) for s in strides])
+        with _on_device_of(block_ids):
             self._check(
                 self._lib.evs_gather_blocks(
                     lp, layer_ptrs.numel(), bp, block_ids.numel(), hp, heads.numel(),
@@ -442,9 +470,9 @@ class Kernels:
         sp = _device_ptr(slots, "scatter_rows: slots", torch.long)
         hp = _device_ptr(heads, "scatter_rows: heads", torch.long)
         _one_device("scatter_rows", layer_ptrs, slots, heads)
-        st = (ctypes.c_int64 * 5)(*[int(s) for s in strides])
+        st = _FIVE(*[int(s) for s in strides])
         n, nl, nh = slots.numel(), layer_ptrs.numel(), heads.numel()
-        with torch.cuda.device(slots.device):
+        with _on_device_of(slots):
             capturing = torch.cuda.is_current_stream_capturing()
             if ordered is None:
                 ordered = sort_first(n, nl, nh, int(d), int(elem_size), capturing, num_slots)
@@ -507,8 +535,8 @@ class Kernels:
         rp = _device_ptr(rows_of, "scatter_pairs: rows_of", torch.long)
         hp = _device_ptr(heads, "scatter_pairs: heads", torch.long)
         _one_device("scatter_pairs", layer_ptrs, slots, rows_of, heads)
-        st = (ctypes.c_int64 * 5)(*[int(s) for s in strides])
-        with torch.cuda.device(slots.device):
+        st = _FIVE(*[int(s) for s in strides])
+        with _on_device_of(slots):
             self._check(
                 self._lib.evs_scatter_pairs(
                     lp, layer_ptrs.numel(), sp, rp, slots.numel(), hp, heads.numel(), int(in_ptr),
@@ -551,8 +579,8 @@ class Kernels:
         fp = _device_ptr(first_rows, "scatter_ranges: first_rows", torch.long)
         hp = _device_ptr(heads, "scatter_ranges: heads", torch.long)
         _one_device("scatter_ranges", layer_ptrs, starts, first_rows, heads)
-        st = (ctypes.c_int64 * 5)(*[int(s) for s in strides])
-        with torch.cuda.device(starts.device):
+        st = _FIVE(*[int(s) for s in strides])
+        with _on_device_of(starts):
             self._check(
                 self._lib.evs_scatter_ranges(
                     lp, layer_ptrs.numel(), sp, fp, starts.numel(), int(num_rows), hp,
@@ -589,7 +617,7 @@ class Kernels:
                 raise RuntimeError(f"order_pairs: {what} holds {t.numel()} entries, not {n}")
         _one_device("order_pairs", slots, out_slots, out_rows)
         need = ctypes.c_int64()
-        with torch.cuda.device(slots.device):
+        with _on_device_of(slots):
             self._check(self._lib.evs_order_pairs_workspace(n, bits, ctypes.byref(need)))
             key = (slots.device, _stream_of(slots.device))
             work = self._workspace.get(key)
@@ -787,7 +815,7 @@ class Kernels:
                                f"words on the device")
         _one_device("local_reduce", bufs, None if isinstance(flags, int) else flags, order, out,
                     state)
-        with torch.cuda.device(out.device):
+        with _on_device_of(out):
             self._check(
                 self._lib.evs_local_reduce(
                     bp, fp, op, out.data_ptr(), out.numel(),
@@ -825,7 +853,7 @@ class Kernels:
         if seqs.dtype != torch.long or not seqs.is_contiguous():
             raise RuntimeError("slot_all_reduce: seqs are contiguous int64")
         _one_device("slot_all_reduce", inp, out, bufs, order, seqs)
-        with torch.cuda.device(inp.device):
+        with _on_device_of(inp):
             self._check(
                 self._lib.evs_slot_all_reduce(
                     inp.data_ptr(), out.data_ptr(), inp.numel(), bp, int(ctrl_ptr),
