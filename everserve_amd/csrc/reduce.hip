@@ -350,6 +350,14 @@ __device__ __forceinline__ void sum_store(const u32x4 (&x)[V][kMaxRows],
   }
 }
 
+// One element of a member's payload, coherent as the vectors are. A global load, not a flat one:
+// member buffers are never LDS.
+__device__ __forceinline__ uint32_t load_element(const uint16_t* p) {
+  if (EVS_REDUCE_FENCE != 3) return *p;
+  return __hip_atomic_load((const __attribute__((address_space(1))) uint16_t*)(p),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The rest of a call from vector vb on: the passes of the vector path, the elements the vectors
 // do not cover, and the completion count (in counting mode C).
 template <int V, int C, bool kCounting = !kControl>
@@ -357,7 +365,8 @@ __device__ __forceinline__ void finish_call(const ReduceArgs& a,
                                             const uint16_t* const (&src)[kMaxRows], int count,
                                             int64_t nvec, int64_t vb, uint64_t* group_word,
                                             uint64_t group_before, uint32_t group,
-                                            uint32_t groups, uint64_t own_outcome) {
+                                            uint32_t groups, uint64_t own_outcome,
+                                            bool tail = true) {
   const int tid = threadIdx.x;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * V;
   // Two-level counting: the group's last workgroup carries the group's outcome to the top word.
@@ -431,19 +440,11 @@ __device__ __forceinline__ void finish_call(const ReduceArgs& a,
   // the elements the vectors do not cover: a tail of fewer than 8, or all of them when a buffer
   // is not 16-byte aligned
   const int64_t first = nvec * 8;
-  for (int64_t e = first + static_cast<int64_t>(blockIdx.x) * kThreads + tid; e < a.n;
+  for (int64_t e = first + static_cast<int64_t>(blockIdx.x) * kThreads + tid; tail && e < a.n;
        e += static_cast<int64_t>(gridDim.x) * kThreads) {
     float acc = 0.0f;
-    for (int q = 0; q < count; q++) {
-      uint32_t b = 0;
-      if (src[q] != nullptr)
-        // a global load, not a flat one: member buffers are never LDS
-        b = EVS_REDUCE_FENCE == 3
-                ? __hip_atomic_load((const __attribute__((address_space(1))) uint16_t*)(src[q] + e),
-                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                : src[q][e];
-      acc += bf16_to_f32(b);
-    }
+    for (int q = 0; q < count; q++)
+      acc += src[q] != nullptr ? bf16_to_f32(load_element(src[q] + e)) : 0.0f;
     a.out[e] = static_cast<uint16_t>(f32_to_bf16(acc));
   }
 
@@ -490,7 +491,7 @@ __device__ __forceinline__ void count_arrival(const ReduceArgs& a, uint64_t* gro
 }
 
 template <int V, int C>
-__global__ __launch_bounds__(kBlockThreads) void local_reduce(ReduceArgs a) {
+__global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a) {
   constexpr bool kStartsEarly = EVS_REDUCE_EARLY && V >= EVS_REDUCE_EARLY_MIN_VPT;
   __shared__ const uint16_t* s_src[kMaxRows];  // member in order position q, or null: missing
   __shared__ int s_count;
@@ -565,6 +566,31 @@ __global__ __launch_bounds__(kBlockThreads) void local_reduce(ReduceArgs a) {
     if (tid >= kThreads) {  // the control wave: it counts, and moves no payload
       if (waiting) __syncthreads();  // the early start's barrier, after wave 0's wait
       if (tid == kThreads) count_arrival<C>(a, group_word, group, groups, s_outcome);
+      // The tail wave, launched where elements are left past the last vector (fewer than 8, one a
+      // lane): it moves them while the payload waves move the vectors. As a round of their own
+      // after those, their loads' round trip and store came at the end of the call. The early start
+      // leaves them to the payload waves, which know the members that came in late. Microseconds
+      // a call in a captured graph, before and now: 16,385 elements of 8 members 3.71 and 3.16
+      // (16,384: 2.90 and 2.88), 119,051 of 8 4.28 and 3.60, 1,420 of 7 3.59 and 2.98. In the
+      // control wave instead, the tail's loads held the count: 119,051 of 8 4.29, 400,007 of 3
+      // 4.32 against 3.91 before.
+      if (tid >= kThreads + 64 && !waiting && (mode & kVectors) != 0 && a.nvec > 0 &&
+          blockIdx.x == gridDim.x - 1) {
+        const int64_t e = a.nvec * 8 + (tid - kThreads - 64);
+        if (e < a.n) {
+          const int members = s_count;
+          uint32_t x[kMaxRows] = {};
+#pragma unroll
+          for (int q = 0; q < kMaxRows; q++) {
+            const uint16_t* p = q < members ? s_src[q] : nullptr;
+            if (p != nullptr) x[q] = load_element(p + e);
+          }
+          float acc = 0.0f;
+#pragma unroll
+          for (int q = 0; q < kMaxRows; q++) acc += bf16_to_f32(x[q]);  // an absent member: +0.0
+          a.out[e] = static_cast<uint16_t>(f32_to_bf16(acc));
+        }
+      }
       return;
     }
   }
@@ -623,7 +649,9 @@ __global__ __launch_bounds__(kBlockThreads) void local_reduce(ReduceArgs a) {
   }
 #endif
 
-  finish_call<V, C>(a, src, count, nvec, vb, group_word, group_before, group, groups, s_outcome);
+  // with vectors, the tail wave has the elements past them
+  finish_call<V, C>(a, src, count, nvec, vb, group_word, group_before, group, groups, s_outcome,
+                    !kControl || nvec == 0);
 }
 
 int64_t g_clock_khz[64];
@@ -696,7 +724,9 @@ extern "C" int evs_local_reduce(const int64_t* bufs, const uint64_t* flags, cons
   if (tail_blocks > blocks) blocks = tail_blocks;
   if (blocks < 1) blocks = 1;
   if (blocks > evs::kMaxBlocks) blocks = evs::kMaxBlocks;
-  const dim3 grid(static_cast<uint32_t>(blocks)), block(evs::kBlockThreads);
+  // one wave more where the vectors leave elements over (see the tail wave)
+  const bool tail = evs::kControl && a.nvec > 0 && a.nvec * 8 < n;
+  const dim3 grid(static_cast<uint32_t>(blocks)), block(evs::kBlockThreads + (tail ? 64 : 0));
   hipStream_t s = evs::as_stream(stream);
   // The counting mode follows the grid. Two-level counting is right for any grid, so the wider
   // kernels, whose grids are past the flat bound whenever the rule above picks them, carry only it.

@@ -101,6 +101,25 @@ def test_the_sum_is_the_ordered_fp32_sum_bit_for_bit(ext, n, order):
     assert not m.state[1:].any()  # the kernel's counters are back at zero
 
 
+@pytest.mark.parametrize("vectors", [1, 255, 256, 257, 9000, 70_000, 140_000])
+@pytest.mark.parametrize("tail", [1, 4, 7])
+@pytest.mark.parametrize("absent", [None, 3])
+def test_the_elements_past_the_last_vector(ext, vectors, tail, absent):
+    """1 to 7 elements past the vectors, in every counting mode and vector width, with every
+    member in and with one that never comes (it sums as zeros)."""
+    n, order = 8 * vectors + tail, [4, 3, 0, 6]
+    inputs = {r: bf16_input(77 * r + n, n) for r in order}
+    m = Members(inputs, order)
+    m.publish(epoch=5, rows=[r for r in order if r != absent])
+    ext.local_reduce(m.bufs, m.flags, m.order, m.out, 5, 10**9 if absent is None else 10**6, 0,
+                     m.state)
+    torch.cuda.synchronize()
+    want = oracle.member_sum([bits(inputs[r]) * (r != absent) for r in order])
+    assert np.array_equal(bits(m.out), want)
+    assert m.status() == ((5, 0, 0) if absent is None else (5, 2, 1 << absent))
+    assert not m.state[1:].any()
+
+
 @pytest.mark.parametrize("n", [3 * (1 << 20) + 5, 6 * (1 << 20)])
 def test_calls_past_the_resident_grid_take_several_passes(ext, n):
     """Past 2 Mi elements the 4-vector kernel's grid stays at 256 workgroups, one a CU with the
