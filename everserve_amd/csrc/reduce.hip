@@ -94,6 +94,9 @@ constexpr int kPollsPerCheck = 32; // flag polls between clock and ABORT reads
 constexpr int kBadOrder = 4;       // reason bit: `order` named a row outside [0, MAX_ROWS)
 constexpr int kVectors = 1;        // mode bit: every member buffer 16-byte aligned
 constexpr int kEarly = 2;          // mode bit: early start (a member missing at the first read)
+constexpr int kFew = 4;            // mode bit: at most kFewMembers listed, and vectors to move
+constexpr int kFewMembers = 4;
+constexpr int kFewPasses = 8;
 constexpr int kDoneBits = 20;      // counting words: workgroups done in bits [0, 20), outcome above
 constexpr uint32_t kGroups = 8;    // group counting words
 // Grids up to this many workgroups count flat, into the top word: their atomics on one address
@@ -274,28 +277,29 @@ __device__ __forceinline__ uint64_t wait_members(const ReduceArgs& a, int lane, 
   return missing;
 }
 
-// The bytes a pass's buffer resources span from vector vb: the vectors left, at most 1 GiB.
+// The bytes a pass's buffer resources span from vector vb: the vectors left, at most 1 GiB (and
+// none past the end).
 __device__ __forceinline__ int pass_records(int64_t nvec, int64_t vb) {
-  const int64_t left = (nvec - vb) * 16;
+  const int64_t left = vb < nvec ? (nvec - vb) * 16 : 0;
   return static_cast<int>(left < (int64_t{1} << 30) ? left : (int64_t{1} << 30));
 }
 
 // One pass's payload loads: vector i of every member q, through q's resource (an absent member's
 // resource is empty, so its loads return zeros without touching memory).
-template <int V>
-__device__ __forceinline__ void load_pass(u32x4 (&x)[V][kMaxRows],
-                                          const __amdgpu_buffer_rsrc_t (&r)[kMaxRows], int tid) {
+template <int V, int Q>
+__device__ __forceinline__ void load_pass(u32x4 (&x)[V][Q],
+                                          const __amdgpu_buffer_rsrc_t (&r)[Q], int tid) {
   // vector-major (1): vector i's loads from every member come before vector i + 1's, so its sum
   // and store can go out while the later vectors' loads are still in flight
 #pragma unroll
-  for (int j = 0; j < V * kMaxRows; j++) {
-    const int i = EVS_REDUCE_LOAD_ORDER ? j / kMaxRows : j % V;
-    const int q = EVS_REDUCE_LOAD_ORDER ? j % kMaxRows : j / V;
+  for (int j = 0; j < V * Q; j++) {
+    const int i = EVS_REDUCE_LOAD_ORDER ? j / Q : j % V;
+    const int q = EVS_REDUCE_LOAD_ORDER ? j % Q : j / V;
     x[i][q] = __builtin_amdgcn_raw_buffer_load_b128(r[q], (i * kThreads + tid) * 16, 0,
                                                     kPayloadScope);
     // keep each vector's loads together, in this order (the scheduler would group them by
     // member otherwise)
-    if (EVS_REDUCE_LOAD_ORDER && q == kMaxRows - 1) __builtin_amdgcn_sched_barrier(0);
+    if (EVS_REDUCE_LOAD_ORDER && q == Q - 1) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -324,8 +328,8 @@ __device__ __forceinline__ void load_late(u32x4 (&x)[V][kMaxRows],
 // through the output resource `ro`, which ends at the last vector, so a store past it is dropped.
 // Adding an absent member's +0.0 changes no sum: the accumulator starts at +0.0 and so is never
 // -0.0. Straight-line, so each vector's sum waits only for its own loads.
-template <int V>
-__device__ __forceinline__ void sum_store(const u32x4 (&x)[V][kMaxRows],
+template <int V, int Q>
+__device__ __forceinline__ void sum_store(const u32x4 (&x)[V][Q],
                                           __amdgpu_buffer_rsrc_t ro, int tid) {
 #pragma unroll
   for (int i = 0; i < V; i++) {
@@ -333,7 +337,7 @@ __device__ __forceinline__ void sum_store(const u32x4 (&x)[V][kMaxRows],
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[e] = 0.0f;
 #pragma unroll
-    for (int q = 0; q < kMaxRows; q++) {
+    for (int q = 0; q < Q; q++) {
 #pragma unroll
       for (int w = 0; w < 4; w++) {
         acc[2 * w] += bf16_to_f32(x[i][q][w] & 0xffffu);
@@ -347,6 +351,41 @@ __device__ __forceinline__ void sum_store(const u32x4 (&x)[V][kMaxRows],
     __builtin_amdgcn_raw_buffer_store_b128(y, ro, (i * kThreads + tid) * 16, 0, kOutputPolicy);
     // the store goes out now, not after the last vector's sum
     if (EVS_REDUCE_LOAD_ORDER) __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// P passes of the first Q order positions (the call lists no more), every pass's loads in flight
+// before the first sum. A pass past the end loads and stores nothing.
+template <int V, int Q, int P>
+__device__ __forceinline__ void pass_group(const uint16_t* const (&src)[kMaxRows], uint16_t* out,
+                                           int64_t nvec, int64_t vb, int64_t stride, int tid) {
+  u32x4 x[P][V][Q];
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int64_t at = vb + p * stride;
+    const int records = pass_records(nvec, at);
+    __amdgpu_buffer_rsrc_t r[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+      r[q] = src[q] != nullptr ? uniform_rsrc(src[q] + at * 8, records) : uniform_rsrc(out, 0);
+    load_pass(x[p], r, tid);
+  }
+#pragma unroll
+  for (int p = 0; p < P; p++) {
+    const int64_t at = vb + p * stride;
+    sum_store(x[p], uniform_rsrc(out + at * 8, pass_records(nvec, at)), tid);
+  }
+}
+
+// Every pass from vector vb on of a call that lists at most Q members, P at a time while more than
+// half as many are left, then fewer.
+template <int V, int Q, int P>
+__device__ __forceinline__ void pass_groups(const uint16_t* const (&src)[kMaxRows], uint16_t* out,
+                                            int64_t nvec, int64_t vb, int64_t stride, int tid) {
+  for (; vb + P / 2 * stride < nvec; vb += P * stride)
+    pass_group<V, Q, P>(src, out, nvec, vb, stride, tid);
+  if constexpr (P > 1) {
+    if (vb < nvec) pass_groups<V, Q, P / 2>(src, out, nvec, vb, stride, tid);
   }
 }
 
@@ -493,6 +532,13 @@ __device__ __forceinline__ void count_arrival(const ReduceArgs& a, uint64_t* gro
 template <int V, int C>
 __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a) {
   constexpr bool kStartsEarly = EVS_REDUCE_EARLY && V >= EVS_REDUCE_EARLY_MIN_VPT;
+  // Few members leave most of a pass's registers empty and few bytes in flight, one workgroup a CU:
+  // the widest kernel then takes several passes at once, in the same registers. Microseconds a
+  // call, one pass at a time and now: two members of 1,200,000 elements 5.67 and 4.48, 3,000,000
+  // 8.68 and 6.37, 33,000,000 49.8 and 36.3; three of 33,000,000 52.2 and 46.1; four of 3,000,000
+  // 9.59 and 8.14. Four members fill the memory's rate by themselves in a long call (33,554,432
+  // elements: 57.2, 57.8 in groups), and keep single passes past kFewPasses.
+  constexpr bool kTakesFew = kControl && EVS_REDUCE_FENCE == 3 && V == kMaxVpt && V > 1;
   __shared__ const uint16_t* s_src[kMaxRows];  // member in order position q, or null: missing
   __shared__ int s_count;
   __shared__ int s_mode;                         // kVectors | kEarly
@@ -541,7 +587,12 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
     }
     if (lane == 0) {
       s_count = count;
-      s_mode = (unaligned ? 0 : kVectors) | (early ? kEarly : 0);
+      const bool few =
+          kTakesFew && !unaligned && a.nvec > 0 &&
+          (count < kFewMembers ||
+           (count == kFewMembers &&
+            a.nvec <= int64_t{kFewPasses} * kMaxBlocks * kThreads * V));
+      s_mode = (unaligned ? 0 : kVectors) | (early ? kEarly : 0) | (few ? kFew : 0);
       s_outcome = (reason << 8) | late_rows;
     }
     // the flags were read with relaxed loads: order the payload reads after them
@@ -606,8 +657,19 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
   if constexpr (kStartsEarly) {
     __shared__ const uint16_t* s_late[kMaxRows];  // member q if it came in during the wait
     __shared__ uint32_t s_came;                     // the order positions s_late names
-    // unlikely: the call whose members are all in at the first read does not run this
-    if (__builtin_expect(waiting, 0)) {
+    // unlikely: a call of many members, all in at the first read, does not run this, and has one
+    // branch here (a second one for the few, in finish_call, cost it 0.1 us of 9.1)
+    if (__builtin_expect((mode & (kEarly | kFew)) != 0, 0)) {
+      if constexpr (kTakesFew) {
+        if (!waiting) {  // the tail wave has the elements past the vectors
+          const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * V;
+          if (__builtin_amdgcn_readfirstlane(count) <= 2)
+            pass_groups<V, 2, 4>(src, a.out, nvec, vb, stride, tid);
+          else
+            pass_groups<V, kFewMembers, 2>(src, a.out, nvec, vb, stride, tid);
+          return;
+        }
+      }
       // The first pass in two rounds of loads: the members that were in at the first read, issued
       // now, and after the wait the members that came in during it. A member that never came in
       // reads as zeros in both. The wait ends on the same events as the one above, so the outcome

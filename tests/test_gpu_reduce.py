@@ -120,6 +120,28 @@ def test_the_elements_past_the_last_vector(ext, vectors, tail, absent):
     assert not m.state[1:].any()
 
 
+@pytest.mark.parametrize("order", [[2], [5, 0], [1, 7, 4], [3, 0, 6, 2]])
+@pytest.mark.parametrize("passes", [0.6, 1.3, 2.6, 3.5, 4.2, 8.1])
+def test_few_members_take_several_passes_at_once(ext, order, passes):
+    """One to four members over part of a pass, one, and group edges (two and four passes at a
+    time, and the passes past which four members go one at a time), with a member that is late
+    from the start in one more call: the ordered fp32 sum bit for bit."""
+    n = int(passes * (1 << 21)) + 3
+    inputs = {r: bf16_input(40 + r, n) for r in order}
+    m = Members(inputs, order)
+    m.publish(epoch=2)
+    ext.local_reduce(m.bufs, m.flags, m.order, m.out, 2, 10**9, 0, m.state)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(m.out), oracle.member_sum([bits(inputs[r]) for r in order]))
+    assert m.status() == (2, 0, 0) and not m.state[1:].any()
+    m.publish(epoch=3, rows=order[:-1])  # the last member never comes
+    ext.local_reduce(m.bufs, m.flags, m.order, m.out, 3, 10**6, 0, m.state)
+    torch.cuda.synchronize()
+    want = oracle.member_sum([bits(inputs[r]) * (r != order[-1]) for r in order])
+    assert np.array_equal(bits(m.out), want)
+    assert m.status() == (3, 2, 1 << order[-1])
+
+
 @pytest.mark.parametrize("n", [3 * (1 << 20) + 5, 6 * (1 << 20)])
 def test_calls_past_the_resident_grid_take_several_passes(ext, n):
     """Past 2 Mi elements the 4-vector kernel's grid stays at 256 workgroups, one a CU with the
