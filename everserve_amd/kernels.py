@@ -53,7 +53,7 @@ ORDER_MIN_SLOTS = 1 << 18
 ORDER_MIN_BYTES = 8 << 30
 """The sizes from which :meth:`Kernels.scatter_rows` sorts its pairs by slot first. Measured on
 MI355X (Llama-3-8B rows, bf16, 16-slot blocks of a permuted table, median of 10 launches), sorted
-against staged order, the sort's 0.11 ms included: every slot of a 262,144-slot cache, 32 layers,
+against staged order, a sort of 0.11 ms included (0.04 since): every slot of a 262,144-slot cache, 32 layers,
 11.58 against 12.17 ms; 8 layers 2.86 against 3.02; 4 layers 1.52 against 1.53; 1 layer 0.47
 against 0.38 (the sort not repaid); a quarter of the cache's blocks, 32 layers, 3.12 against 3.08
 (writes spread over a sparse part of a cache gain nothing from order). The call cannot see the
