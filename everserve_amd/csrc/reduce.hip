@@ -537,7 +537,8 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
   // call, one pass at a time and now: two members of 1,200,000 elements 5.67 and 4.48, 3,000,000
   // 8.68 and 6.37, 33,000,000 49.8 and 36.3; three of 33,000,000 52.2 and 46.1; four of 3,000,000
   // 9.59 and 8.14. Four members fill the memory's rate by themselves in a long call (33,554,432
-  // elements: 57.2, 57.8 in groups), and keep single passes past kFewPasses.
+  // elements: 57.2, 57.8 in groups), and take single passes past kFewPasses, of four members'
+  // loads instead of eight (20,000,000 elements 36.9 and 35.9, 33,554,432 58.0 and 57.7).
   constexpr bool kTakesFew = kControl && EVS_REDUCE_FENCE == 3 && V == kMaxVpt && V > 1;
   __shared__ const uint16_t* s_src[kMaxRows];  // member in order position q, or null: missing
   __shared__ int s_count;
@@ -587,11 +588,7 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
     }
     if (lane == 0) {
       s_count = count;
-      const bool few =
-          kTakesFew && !unaligned && a.nvec > 0 &&
-          (count < kFewMembers ||
-           (count == kFewMembers &&
-            a.nvec <= int64_t{kFewPasses} * kMaxBlocks * kThreads * V));
+      const bool few = kTakesFew && !unaligned && a.nvec > 0 && count <= kFewMembers;
       s_mode = (unaligned ? 0 : kVectors) | (early ? kEarly : 0) | (few ? kFew : 0);
       s_outcome = (reason << 8) | late_rows;
     }
@@ -665,8 +662,11 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
           const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * V;
           if (__builtin_amdgcn_readfirstlane(count) <= 2)
             pass_groups<V, 2, 4>(src, a.out, nvec, vb, stride, tid);
-          else
+          else if (__builtin_amdgcn_readfirstlane(count) < kFewMembers ||
+                   nvec <= kFewPasses * stride)
             pass_groups<V, kFewMembers, 2>(src, a.out, nvec, vb, stride, tid);
+          else
+            pass_groups<V, kFewMembers, 1>(src, a.out, nvec, vb, stride, tid);
           return;
         }
       }
