@@ -404,8 +404,7 @@ __device__ __forceinline__ void finish_call(const ReduceArgs& a,
                                             const uint16_t* const (&src)[kMaxRows], int count,
                                             int64_t nvec, int64_t vb, uint64_t* group_word,
                                             uint64_t group_before, uint32_t group,
-                                            uint32_t groups, uint64_t own_outcome,
-                                            bool tail = true) {
+                                            uint32_t groups, uint64_t own_outcome, bool tail) {
   const int tid = threadIdx.x;
   const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * V;
   // Two-level counting: the group's last workgroup carries the group's outcome to the top word.
@@ -542,8 +541,9 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
   constexpr bool kTakesFew = kControl && EVS_REDUCE_FENCE == 3 && V == kMaxVpt && V > 1;
   __shared__ const uint16_t* s_src[kMaxRows];  // member in order position q, or null: missing
   __shared__ int s_count;
-  __shared__ int s_mode;                         // kVectors | kEarly
+  __shared__ int s_mode;                         // kVectors | kEarly | kFew
   __shared__ uint32_t s_outcome;                 // reason << 8 | late rows
+  __shared__ const uint16_t* s_late[kMaxRows];   // early start: member q if it came in later
 
   const int tid = threadIdx.x;
   const int64_t first_vb = static_cast<int64_t>(blockIdx.x) * kThreads * V;  // first vector
@@ -616,13 +616,15 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
       if (tid == kThreads) count_arrival<C>(a, group_word, group, groups, s_outcome);
       // The tail wave, launched where elements are left past the last vector (fewer than 8, one a
       // lane): it moves them while the payload waves move the vectors. As a round of their own
-      // after those, their loads' round trip and store came at the end of the call. The early start
-      // leaves them to the payload waves, which know the members that came in late. Microseconds
+      // after those, their loads' round trip and store came at the end of the call. The last
+      // workgroup's has them alone, whether it starts early or not: workgroups may differ in that
+      // (a flag can land between two workgroups' first reads), so no rule that asks how a
+      // workgroup started gives the elements exactly one owner. Microseconds
       // a call in a captured graph, before and now: 16,385 elements of 8 members 3.71 and 3.16
       // (16,384: 2.90 and 2.88), 119,051 of 8 4.28 and 3.60, 1,420 of 7 3.59 and 2.98. In the
       // control wave instead, the tail's loads held the count: 119,051 of 8 4.29, 400,007 of 3
       // 4.32 against 3.91 before.
-      if (tid >= kThreads + 64 && !waiting && (mode & kVectors) != 0 && a.nvec > 0 &&
+      if (tid >= kThreads + 64 && (mode & kVectors) != 0 && a.nvec > 0 &&
           blockIdx.x == gridDim.x - 1) {
         const int64_t e = a.nvec * 8 + (tid - kThreads - 64);
         if (e < a.n) {
@@ -631,6 +633,7 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
 #pragma unroll
           for (int q = 0; q < kMaxRows; q++) {
             const uint16_t* p = q < members ? s_src[q] : nullptr;
+            if (waiting && p == nullptr) p = s_late[q];  // null past the members too
             if (p != nullptr) x[q] = load_element(p + e);
           }
           float acc = 0.0f;
@@ -652,13 +655,12 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
   for (int q = 0; q < kMaxRows; q++) src[q] = q < count ? s_src[q] : nullptr;
 #if EVS_REDUCE_EARLY
   if constexpr (kStartsEarly) {
-    __shared__ const uint16_t* s_late[kMaxRows];  // member q if it came in during the wait
-    __shared__ uint32_t s_came;                     // the order positions s_late names
+    __shared__ uint32_t s_came;  // the order positions s_late names
     // unlikely: a call of many members, all in at the first read, does not run this, and has one
     // branch here (a second one for the few, in finish_call, cost it 0.1 us of 9.1)
     if (__builtin_expect((mode & (kEarly | kFew)) != 0, 0)) {
       if constexpr (kTakesFew) {
-        if (!waiting) {  // the tail wave has the elements past the vectors
+        if (!waiting) {
           const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads * V;
           if (__builtin_amdgcn_readfirstlane(count) <= 2)
             pass_groups<V, 2, 4>(src, a.out, nvec, vb, stride, tid);
@@ -699,13 +701,13 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
       load_late(x, s_late, __builtin_amdgcn_readfirstlane(s_came), vb, records, tid);
       sum_store(x, uniform_rsrc(a.out + vb * 8, records), tid);
       vb += static_cast<int64_t>(gridDim.x) * kThreads * V;
-      // the later passes and the element tail read every member that is in; this path ends here,
-      // so the common path's code stays as it is
+      // the later passes read every member that is in; this path ends here, so the common path's
+      // code stays as it is
 #pragma unroll
       for (int q = 0; q < kMaxRows; q++)
         if (src[q] == nullptr) src[q] = s_late[q];
       finish_call<V, C>(a, src, count, nvec, vb, group_word, group_before, group, groups,
-                        s_outcome);
+                        s_outcome, !kControl);
       return;
     }
   }

@@ -142,6 +142,78 @@ def test_few_members_take_several_passes_at_once(ext, order, passes):
     assert m.status() == (3, 2, 1 << order[-1])
 
 
+@pytest.mark.parametrize("order", [[3, 0], [2, 6, 0, 5], [5, 3, 7, 0, 1, 6, 2, 4]])
+@pytest.mark.parametrize("n", [8 * 70_000 + 5, 8 * 140_000 + 1, 3_000_007])
+def test_a_flag_that_lands_while_the_workgroups_start(ext, order, n):
+    """A member's flag is written 0 to 30 us after the launch call, and every other time with
+    another stream's copy on the CUs, so that it lands between the workgroups' first reads of the
+    flags: some find the member in and some start early (two launches of three; in one of forty
+    the last workgroup starts early and the first does not). Whatever the mix, every element is
+    written, those past the last vector too: ``out`` is filled with a pattern first."""
+    flags_host, flags_dev = ext.host_alloc_mapped(MAXW * 8)
+    try:
+        words = (ctypes.c_int64 * MAXW).from_address(flags_host)
+        inputs = {r: bf16_input(90 + r, n) for r in order}
+        m = Members(inputs, order)
+        want = torch.from_numpy(oracle.member_sum([bits(inputs[r]) for r in order])
+                                .view(np.int16)).cuda()
+        unwritten = 0x7F5A  # a NaN no rounding gives
+        late, side = order[1], torch.cuda.Stream()
+        busy = torch.zeros((2, 16 << 20), dtype=torch.int32, device="cuda")
+        for i in range(120):
+            epoch = i + 1
+            m.out.view(torch.int16).fill_(unwritten)
+            for r in order:
+                words[r] = epoch - 1 if r == late else epoch
+            torch.cuda.synchronize()
+            if i % 2:
+                with torch.cuda.stream(side):
+                    busy[0].copy_(busy[1])
+            ext.local_reduce(m.bufs, flags_dev, m.order, m.out, epoch, 3_000_000_000, 0, m.state)
+            release = time.perf_counter_ns() + (i // 2) * 500
+            while time.perf_counter_ns() < release:
+                pass
+            words[late] = epoch
+            torch.cuda.synchronize()
+            got = m.out.view(torch.int16)
+            wrong = torch.nonzero(got != want)
+            assert not wrong.numel(), (i, wrong.flatten().tolist()[:8], got[-8:].tolist())
+            assert m.status() == (epoch, 0, 0) and not m.state[1:].any()
+    finally:
+        ext.host_free(flags_host)
+
+
+@pytest.mark.parametrize("order", [[2], [5, 0], [1, 7, 4], [3, 0, 6, 2]])
+@pytest.mark.parametrize("n", [(1 << 20) + 11, int(2.6 * (1 << 21)) + 3])
+def test_few_members_one_of_which_arrives_mid_wait(ext, order, n):
+    """One to four members, the last of which is named late and then arrives: part of a pass and
+    several, with elements past the last vector."""
+    flags_host, flags_dev = ext.host_alloc_mapped(MAXW * 8)
+    ctrl = Ctrl(ext)
+    try:
+        words = (ctypes.c_int64 * MAXW).from_address(flags_host)
+        inputs = {r: bf16_input(20 + r, n) for r in order}
+        m = Members(inputs, order)
+        m.out.zero_()
+        for r in order:
+            words[r] = 0 if r == order[-1] else 4
+        torch.cuda.synchronize()
+        ctrl.words[BOUND] = 100_000
+        ext.local_reduce(m.bufs, flags_dev, m.order, m.out, 4, 3_000_000_000, ctrl.dev, m.state)
+        try:
+            waited = named(ctrl, 1 << order[-1])
+        finally:
+            words[order[-1]] = 4
+        torch.cuda.synchronize()
+        assert waited, "the call never named the last member: it did not wait for it"
+        assert np.array_equal(bits(m.out), oracle.member_sum([bits(inputs[r]) for r in order]))
+        assert m.status() == (4, 0, 0) and not m.state[1:].any()
+        assert int(ctrl.words[LATE]) == 0
+    finally:
+        ctrl.close()
+        ext.host_free(flags_host)
+
+
 @pytest.mark.parametrize("n", [3 * (1 << 20) + 5, 6 * (1 << 20)])
 def test_calls_past_the_resident_grid_take_several_passes(ext, n):
     """Past 2 Mi elements the 4-vector kernel's grid stays at 256 workgroups, one a CU with the
