@@ -277,7 +277,7 @@ _HERE = contextlib.nullcontext()
 
 
 def _stream_of(device) -> int:
-    """The handle of torch's current stream of ``device``."""
+    """The handle of torch's current stream of ``device``, a ``torch.device`` of a GPU."""
     import torch
 
     index = device.index
@@ -637,10 +637,15 @@ class Kernels:
         current stream (device to host into pinned memory, or host to device)."""
         import torch
 
-        dev = device if device is not None else torch.device("cuda", torch.cuda.current_device())
+        if device is None:
+            stream = _stream_of(torch.device("cuda", torch.cuda.current_device()))
+        elif isinstance(device, torch.device) and device.type == "cuda":
+            stream = _stream_of(device)
+        else:  # an index or a name; what is no GPU is refused
+            stream = torch.cuda.current_stream(device).cuda_stream
         self._check(
             self._lib.evs_copy_rows_async(int(dst_ptr), int(src_ptr), int(groups), int(bytes_),
-                                          int(pitch), _stream_of(dev))
+                                          int(pitch), stream)
         )
 
     def host_gather_ranges(self, src_ptr: int, src_rows: int, row_bytes: int, starts, counts,

@@ -74,3 +74,28 @@ def test_without_a_gpu_the_kernels_do_not_load():
 def test_a_build_names_the_gpus_it_runs_on():
     assert kernels.built_archs("gfx942;gfx950") == {"gfx942", "gfx950"}
     assert kernels.built_archs("gfx950:sramecc+:xnack- gfx942") == {"gfx950", "gfx942"}
+
+
+def test_a_copys_device_is_whatever_torch_takes_for_one(monkeypatch):
+    """An index, a name, a device with or without an index, or none: the current stream of that
+    GPU; a device that is no GPU is refused."""
+    import types
+
+    import torch
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "_lazy_init", lambda: None)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 100 + index)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentStream", lambda index: (100 + index, index, 1))
+    monkeypatch.setattr(torch.cuda, "Stream", lambda stream_id, device_index, device_type:
+                        types.SimpleNamespace(cuda_stream=stream_id))
+    streams = []
+    ext = types.SimpleNamespace(
+        _check=lambda rc: None,
+        _lib=types.SimpleNamespace(evs_copy_rows_async=lambda *args: streams.append(args[-1])))
+    for device in (None, torch.device("cuda"), 0, 2, "cuda:1", torch.device("cuda", 1)):
+        kernels.Kernels.copy_rows_async(ext, 1 << 20, 1 << 21, 2, 16, 32, device)
+    assert streams == [103, 103, 100, 102, 101, 101]
+    for device in ("cpu", torch.device("cpu"), torch.device("meta")):
+        with pytest.raises(ValueError, match="cuda device"):
+            kernels.Kernels.copy_rows_async(ext, 1 << 20, 1 << 21, 2, 16, 32, device)
