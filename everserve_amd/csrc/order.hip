@@ -390,9 +390,11 @@ int tiles_of(int64_t n) {
   return static_cast<int>((n + tile - 1) / tile);
 }
 
-// The radix sort's workspace: the pairs between passes, the counts and the ORs.
+// The radix sort's workspace: the pairs between passes, the counts and the ORs. Sized for the
+// smaller tile at every size, though a sort past 2^19 pairs has half as many, so that it grows with
+// the pairs: a workspace for a caller's largest call holds its smaller ones.
 int64_t sorted_bytes(int64_t n) {
-  const int64_t tiles = tiles_of(n);
+  const int64_t tiles = (n + tile_pairs(4) - 1) / tile_pairs(4);
   return 2 * round_up(n * 8) + round_up(tiles * kBins * 2) + round_up(tiles * 8);
 }
 

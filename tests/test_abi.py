@@ -144,3 +144,18 @@ def test_scatter_rows_sorts_first_from_two_to_the_18_slots_and_8_gib():
     assert sf(1 << 18, capturing=False, num_slots=1 << 18, **c4)
     assert sf(7 << 17, capturing=False, num_slots=1 << 20, **c4)
     assert not sf((7 << 17) - 1, capturing=False, num_slots=1 << 20, **c4)
+
+
+@pytest.mark.parametrize("bits", [1, 18, 64])
+def test_the_orders_workspace_grows_with_the_pairs(lib, bits):
+    """A caller that sizes the workspace for its largest call may use it for every smaller one:
+    the bytes never fall as the pairs grow, over each place where the sort changes its tiles."""
+    edges = [2048, 8192, 1 << 18, 1 << 19, 532_384, 1 << 20]
+    sizes = sorted({0, 1, *(e + d for e in edges for d in range(-3, 4)), *range(1, 1 << 20, 4099)})
+    sizes = [n for n in sizes if n <= 1 << 20]  # past it the sort asks the device
+    need, got = ctypes.c_int64(), []
+    for n in sizes:
+        assert lib.evs_order_pairs_workspace(n, bits, ctypes.byref(need)) == 0
+        got.append(need.value)
+    falls = [(a, b) for a, b, x, y in zip(sizes, sizes[1:], got, got[1:]) if y < x]
+    assert not falls, falls
