@@ -114,6 +114,50 @@ def test_words_narrower_than_16_bytes(ext, layout, dtype, d, shift):
 
 
 @pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("dtype,d", [(torch.float8_e4m3fn, 120), (torch.float8_e4m3fn, 126),
+                                     (torch.bfloat16, 100), (torch.float32, 6)])
+@pytest.mark.parametrize("shift", [0, 1, 3])
+def test_bases_off_the_word_by_blocks_pairs_and_ranges(ext, layout, dtype, d, shift):
+    """The block gather, the pair scatter and the range scatter over layers whose bases lie
+    ``shift`` elements into their storage, as many 8-, 4- or 2-byte words do not fit."""
+    blocks, heads = [9, 0, 77, 40], [2, 0]
+    n = len(blocks) * BS
+    layers = caches(layout, d, dtype, n_layers=L, nb=NB, h=H, seed=d + shift)
+    slots = [b * BS + i for b in blocks for i in range(BS)]
+    e, st = layers[0].element_size(), strides_of(layers[0])
+    want = oracle.gather_rows(layers, slots, heads, n, d, BS, st, e)
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + shift, dtype=t.dtype, device="cuda")
+        return flat[shift:].view(t.shape).copy_(t)
+
+    gpu = [shifted(t) for t in layers]
+    out = torch.zeros(want.nbytes, dtype=torch.uint8, device="cuda")
+    ext.gather_blocks(ptrs(gpu), torch.tensor(blocks, dtype=torch.int32, device="cuda"),
+                      dev_long(heads), out.data_ptr(), n, d, BS, list(st), e)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy().view(want.dtype).reshape(want.shape), want)
+
+    perm = np.random.default_rng(d).permutation(n)
+    for by_ranges in (False, True):
+        dst = caches(layout, d, dtype, n_layers=L, nb=NB, h=H, seed=d + 7)
+        gpu = [shifted(t) for t in dst]
+        if by_ranges:
+            oracle.scatter_rows(dst, slots, heads, want, n, d, BS, st, e)
+            ext.scatter_ranges(ptrs(gpu), dev_long([b * BS for b in blocks]),
+                               dev_long(range(0, n + 1, BS)), n, dev_long(heads), out.data_ptr(),
+                               n, d, BS, list(st), e)
+        else:
+            oracle.scatter_rows(dst, slots, heads, np.ascontiguousarray(want[:, :, perm]), n, d,
+                                BS, st, e)
+            ext.scatter_pairs(ptrs(gpu), dev_long(slots), dev_long(perm), dev_long(heads),
+                              out.data_ptr(), n, d, BS, list(st), e)
+        torch.cuda.synchronize()
+        for g, w in zip(gpu, dst):
+            assert np.array_equal(bits(g), bits(w))
+
+
+@pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("heads_total", [2, 5, 8, 12])
 @pytest.mark.parametrize("dtype,d", [(torch.float8_e4m3fn, 64), (torch.float8_e4m3fn, 96),
                                      (torch.float8_e4m3fn, 120), (torch.bfloat16, 80),
