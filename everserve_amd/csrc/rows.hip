@@ -186,14 +186,25 @@ constexpr int threads_of(int d, int i, int form = kPlain) {
          : form == kSpanning  ? 256
                               : EVS_SCATTER_THREADS;
 }
-// A narrower word's passes and tiles hold more of them: 2x at 8 bytes (the same bytes a tile), 4x
-// below, where the work is the address arithmetic a word takes. 400 MB gathered from one head, 4x
-// and 2x against 1x: 8-byte words (bf16 100) 5,507 and 5,467 against 3,670 GB/s, 2-byte words
-// (fp8 126) 3,433 and 2,428 against 1,546; (bf16 124, 8-byte) 4,286 and 5,516 against 4,560.
+// A narrower word's tiles hold more of them: 2x at 8 bytes (the same bytes a tile), 4x
+// below, where the work is the address arithmetic a word
+// takes. 400 MB gathered from one head, 4x and 2x against 1x: 8-byte words (bf16 100) 5,507 and
+// 5,467 against 3,670 GB/s, 2-byte words (fp8 126) 3,433 and 2,428 against 1,546; (bf16 124,
+// 8-byte) 4,286 and 5,516 against 4,560.
 constexpr int narrow_of(size_t word) { return word == 16 ? 1 : word == 8 ? 2 : 4; }
+constexpr int base_vpt(int d, int i) {
+  return i == kByPairs ? EVS_PAIRS_VPT : d == kGather ? EVS_GATHER_VPT : EVS_SCATTER_VPT;
+}
+// Words a thread and pass: the gather's as many times more, and the slot and range scatters' of
+// 4-byte words; the other scatters' passes, and the pair scatter's tiles, at most twice as many.
+// Microseconds for 8 layers of 4,096 slots of 8 heads, four times, twice, and by elements in a
+// 16-byte word's tiles: pairs, bf16 121 215, 137 and 140, fp8 126 116, 79 and 125; slots, bf16 121
+// 181, 140 and 197; ranges 216, 163 and 277; but slots of 4-byte words (bf16 126) 80 and 86. Four
+// times as many words a pair tile ran 39.5 against 43.7 (fp8 100, kv_first), but 59.5 against 46.5
+// in the combined layout.
 constexpr int vpt_of(int d, int i, size_t word) {
-  return narrow_of(word) *
-         (i == kByPairs ? EVS_PAIRS_VPT : d == kGather ? EVS_GATHER_VPT : EVS_SCATTER_VPT);
+  const bool most = d == kGather || (i != kByPairs && word == 4);
+  return base_vpt(d, i) * (most ? narrow_of(word) : word == 16 ? 1 : 2);
 }
 constexpr int nt_of(int d, int i) {
   return i == kByPairs    ? EVS_PAIRS_NT
@@ -493,6 +504,48 @@ __device__ __forceinline__ void gather_by_halves(uint32_t v0, uint32_t wave, uin
     gather_by_halves<kWords / 2, T, kThreads, kNt>(v0, wave, words, locate);
 }
 
+// Move a scatter's tile of `words` words, kWords a thread and pass; those locate() has no place for
+// move nothing.
+template <int kWords, typename T, int D, int I, int F, typename Locate>
+__device__ __forceinline__ void scatter_words(uint32_t words, const Locate& locate) {
+  constexpr int kThreads = threads_of(D, I, F);
+  for (uint32_t v0 = 0; v0 < words; v0 += kThreads * kWords) {
+    // The slot scatter waits for each load before the next: its stores land in a random order,
+    // and fewer accesses in flight ran faster (65,536 permuted slots x 4 layers x 8 bf16 heads
+    // of 128: 5,764 GB/s, 5,620 with a thread's loads in flight together, 5,746 with the last
+    // load not waited for). The range and pair scatters, whose stores run along the cache, ran
+    // slower so (5,207 against 5,602 and 5,790 against 5,837), and keep their loads together, as
+    // does the slot scatter that spans heads (bf16 112, 8 heads: 5,235 against 4,908).
+    T w[kWords];
+    char* src[kWords];
+    char* dst[kWords];
+    bool live[kWords];
+#pragma unroll
+    for (int i = 0; i < kWords; i++)
+      live[i] = locate(v0 + i * kThreads + threadIdx.x, dst[i], src[i]);
+#pragma unroll
+    for (int i = 0; i < kWords; i++) {
+      if (live[i]) w[i] = load_word<T, kStaged, (nt_of(D, I) & 1) != 0>(src[i]);
+      if (I == kBySlots && F == kPlain) __builtin_amdgcn_s_waitcnt(kVmcntZero);
+    }
+#pragma unroll
+    for (int i = 0; i < kWords; i++)
+      if (live[i]) store_word<T, kCache, (nt_of(D, I) & 2) != 0>(dst[i], w[i]);
+  }
+}
+
+// The same in passes no wider than the tile needs.
+template <int kWords, typename T, int D, int I, int F, typename Locate>
+__device__ __forceinline__ void scatter_passes(uint32_t words, const Locate& locate) {
+  if constexpr (kWords > base_vpt(D, I)) {
+    if (words <= threads_of(D, I, F) * kWords / 2) {
+      scatter_passes<kWords / 2, T, D, I, F>(words, locate);
+      return;
+    }
+  }
+  scatter_words<kWords, T, D, I, F>(words, locate);
+}
+
 // Move one tile's words: the slots' offsets and the heads' are in LDS, and for the pair scatter
 // the staged rows'. A wave past the tile's last word leaves; in the wave that holds the last word
 // the gather's lanes past it move that word again, which costs nothing (the same lines in the
@@ -555,31 +608,7 @@ __device__ __forceinline__ void move_tile(const RowsArgs& a, const int64_t* s_sl
     }
     return;
   }
-  for (uint32_t v0 = 0; v0 < words; v0 += kThreads * kVpt) {
-    // The slot scatter waits for each load before the next: its stores land in a random order,
-    // and fewer accesses in flight ran faster (65,536 permuted slots x 4 layers x 8 bf16 heads
-    // of 128: 5,764 GB/s, 5,620 with a thread's loads in flight together, 5,746 with the last
-    // load not waited for). The range and pair scatters, whose stores run along the cache, ran
-    // slower so (5,207 against 5,602 and 5,790 against 5,837), and keep their loads together, as
-    // does the slot scatter that spans heads (bf16 112, 8 heads: 5,235 against 4,908).
-    T w[kVpt];
-    char* src[kVpt];
-    char* dst[kVpt];
-    bool live[kVpt];
-#pragma unroll
-    for (int i = 0; i < kVpt; i++) {
-      const uint32_t v = v0 + i * kThreads + tid;
-      live[i] = locate(v, dst[i], src[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < kVpt; i++) {
-      if (live[i]) w[i] = load_word<T, kStaged, (nt_of(D, I) & 1) != 0>(src[i]);
-      if (I == kBySlots && F == kPlain) __builtin_amdgcn_s_waitcnt(kVmcntZero);
-    }
-#pragma unroll
-    for (int i = 0; i < kVpt; i++)
-      if (live[i]) store_word<T, kCache, (nt_of(D, I) & 2) != 0>(dst[i], w[i]);
-  }
+  scatter_passes<kVpt, T, D, I, F>(words, locate);
 }
 
 // Fill a tile's slot and head offsets into LDS. The first wave reads both index entries before it
@@ -666,7 +695,7 @@ constexpr int64_t kLine = 128;
 int64_t per_line(int64_t bytes) { return kLine / std::gcd(kLine, bytes); }
 
 // Launch tiles of `hg` heads (0: all) and about `target` words. lines: a gather's tile may be cut
-// or grown to whole lines of its rows.
+// or grown to whole lines of its rows, and a call past the launch limit is tried in plain tiles.
 template <int D, int I, int F, typename T>
 int launch_tiles(RowsArgs a, int64_t L, int64_t hg, int64_t target, hipStream_t stream,
                  const char* name, bool lines = true) {
@@ -702,12 +731,18 @@ int launch_tiles(RowsArgs a, int64_t L, int64_t hg, int64_t target, hipStream_t 
   EVS_REQUIRE(ts * per_slot < (int64_t{1} << 31), "%s: a tile of %lld words is too large", name,
               static_cast<long long>(ts * per_slot));
   // HIP on AMD GPUs takes at most 2^32 - 1 work-items along x (gridDim.x * blockDim.x). A shape
-  // chosen for its lines may leave some of a tile's words empty, and so need more workgroups: a
-  // call that is too large for it still fits the plain one.
-  if (I != kByPairs && lines && grid * threads >= (int64_t{1} << 32))
+  // chosen for its lines may leave some of a tile's words empty, and so need more workgroups, and
+  // the pair scatter's tiles hold no more than twice a 16-byte word's: a call that is too large for
+  // them still fits the plain ones.
+  if (lines && grid * threads >= (int64_t{1} << 32))
     return launch_tiles<D, I, kPlain, T>(
-        a, L, D == kGather ? EVS_GATHER_HEADS_PER_TILE : EVS_SCATTER_HEADS_PER_TILE,
-        (D == kGather ? EVS_GATHER_TILE_WORDS : EVS_SCATTER_TILE_WORDS) * narrow_of(sizeof(T)),
+        a, L,
+        I == kByPairs    ? EVS_PAIRS_HEADS_PER_TILE
+        : D == kGather ? EVS_GATHER_HEADS_PER_TILE
+                       : EVS_SCATTER_HEADS_PER_TILE,
+        (I == kByPairs    ? EVS_PAIRS_TILE_WORDS
+         : D == kGather ? EVS_GATHER_TILE_WORDS
+                        : EVS_SCATTER_TILE_WORDS) * narrow_of(sizeof(T)),
         stream, name, false);
   EVS_REQUIRE(grid * threads < (int64_t{1} << 32),
               "%s: %lld workgroups of %d threads exceed the launch limit of 2^32 - 1 work-items; "
@@ -773,8 +808,9 @@ int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const ch
   a.W = W;
   constexpr int64_t kNarrow = narrow_of(sizeof(T));
   if constexpr (I == kByPairs) {
+    constexpr int64_t kTwice = kNarrow < 2 ? kNarrow : 2;  // at most (see vpt_of)
     return launch_tiles<D, I, kPlain, T>(a, L, EVS_PAIRS_HEADS_PER_TILE,
-                                        EVS_PAIRS_TILE_WORDS * kNarrow, stream, name);
+                                        EVS_PAIRS_TILE_WORDS * kTwice, stream, name);
   } else if constexpr (D == kGather) {
     constexpr int64_t target = EVS_GATHER_TILE_WORDS * kNarrow;
     const int64_t hg = gather_heads(a, target);
