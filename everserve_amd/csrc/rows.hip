@@ -113,6 +113,7 @@ namespace {
 #define EVS_RANGES_XCD_CHUNK -1
 #endif
 constexpr uint32_t kXcds = 8;
+constexpr int64_t kCUs = 256;
 // The pair scatter (a staged row per listed slot, listed in the order the caller wants written):
 // its tiles span all heads (2 slots x 8 heads at bf16 d=128, 8 KiB) and its words run along the
 // cache, so that a caller listing its slots in increasing order writes each layer's cache front
@@ -186,8 +187,8 @@ constexpr int threads_of(int d, int i, int form = kPlain) {
          : form == kSpanning  ? 256
                               : EVS_SCATTER_THREADS;
 }
-// A narrower word's tiles hold more of them: 2x at 8 bytes (the same bytes a tile), 4x
-// below, where the work is the address arithmetic a word
+// A narrower word's tiles hold more of them where the call is large enough (see tile_words): up to
+// 2x at 8 bytes (the same bytes a tile), 4x below, where the work is the address arithmetic a word
 // takes. 400 MB gathered from one head, 4x and 2x against 1x: 8-byte words (bf16 100) 5,507 and
 // 5,467 against 3,670 GB/s, 2-byte words (fp8 126) 3,433 and 2,428 against 1,546; (bf16 124,
 // 8-byte) 4,286 and 5,516 against 4,560.
@@ -534,7 +535,8 @@ __device__ __forceinline__ void scatter_words(uint32_t words, const Locate& loca
   }
 }
 
-// The same in passes no wider than the tile needs.
+// The same in passes no wider than such a tile needs: a small call's holds one pass of a 16-byte
+// word's.
 template <int kWords, typename T, int D, int I, int F, typename Locate>
 __device__ __forceinline__ void scatter_passes(uint32_t words, const Locate& locate) {
   if constexpr (kWords > base_vpt(D, I)) {
@@ -803,17 +805,36 @@ int64_t span_heads(const RowsArgs& a, int64_t target) {
   return best;
 }
 
+// Sizes of a call, in words, at which its tiles change: below them a larger tile leaves a CU so
+// few waves that their own round trips are the call's time. From kTwice on the tiles of narrow
+// words hold twice a 16-byte word's number, from kFourTimes (words below 8 bytes) four times.
+// Below kFewWords a gather's tile has two heads at most. Microseconds with the large tiles at
+// every size, and so: gathers of 8 slots of 8 heads of one layer, fp8 120 3.85 and 2.64, bf16 120
+// 3.32 and 2.62; 16 slots x 32 layers 4.22 and 2.81, 3.60 and 2.85; the scatter's 8 slots of 8 fp8
+// heads of 120 3.12 and 2.66. Calls past each line ran as fast or faster in the larger tiles (0.4
+// to 3.5 million words of every width, each 1x, 2x and 4x).
+constexpr int64_t kFewWords = 1024 * kCUs;
+constexpr int64_t kTwice = 2048 * kCUs;
+constexpr int64_t kFourTimes = 8192 * kCUs;
+
+// The words a tile aims at in a call of `words`, with `base` a 16-byte word's.
+template <typename T>
+int64_t tile_words(int64_t base, int64_t words) {
+  const int64_t times = words >= kFourTimes ? 4 : words >= kTwice ? 2 : 1;
+  return base * (times < narrow_of(sizeof(T)) ? times : narrow_of(sizeof(T)));
+}
+
 template <int D, int I, typename T>
 int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const char* name) {
   a.W = W;
-  constexpr int64_t kNarrow = narrow_of(sizeof(T));
+  const int64_t words = L * a.H * a.n * 2 * W;
   if constexpr (I == kByPairs) {
-    constexpr int64_t kTwice = kNarrow < 2 ? kNarrow : 2;  // at most (see vpt_of)
+    const int64_t twice = words < kFourTimes ? words : kTwice;  // at most (see vpt_of)
     return launch_tiles<D, I, kPlain, T>(a, L, EVS_PAIRS_HEADS_PER_TILE,
-                                        EVS_PAIRS_TILE_WORDS * kTwice, stream, name);
+                                        tile_words<T>(EVS_PAIRS_TILE_WORDS, twice), stream, name);
   } else if constexpr (D == kGather) {
-    constexpr int64_t target = EVS_GATHER_TILE_WORDS * kNarrow;
-    const int64_t hg = gather_heads(a, target);
+    const int64_t target = tile_words<T>(EVS_GATHER_TILE_WORDS, words);
+    const int64_t hg = words < kFewWords ? EVS_GATHER_HEADS_PER_TILE : gather_heads(a, target);
     if constexpr (sizeof(T) == 16) {
       // Two heads a tile of several (their rows far apart, see gather_heads), in whole lines: half
       // the tile. bf16 heads of 128, 32 layers, 8 heads: 16,384 slots 6,179 against 6,168 GB/s,
@@ -829,13 +850,17 @@ int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const ch
     // instead, one slot's heads after another. 400 MB, 8 heads, by slots: fp8 64 4,519 -> 5,630
     // GB/s, 96 2,220 -> 5,290, 120 1,910 -> 4,627, bf16 80 2,950 -> 5,358, 112 3,498 -> 5,235, 120
     // 3,104 -> 5,347; by 1,034 ranges: fp8 64 3,823 -> 5,423, bf16 80 2,834 -> 4,921. Half-rows of
-    // whole lines run faster one head a tile (bf16 128: 5,862 against 5,627 spanning).
+    // whole lines run faster one head a tile (bf16 128: 5,862 against 5,627 spanning). A slot whose
+    // heads do not fit one pass spans only where such slots fill the CUs twice: 18 slots x 8 layers
+    // of 16 bf16 heads of 121 took 6.6 us spanning and take 4.4, 64 slots 7.2 and 7.0.
     if (a.H > 1 && a.sh == a.half_bytes && per_line(a.half_bytes) > 1) {
-      constexpr int64_t target = 512 * kNarrow;  // one pass of the 256 threads
-      return launch_tiles<D, I, kSpanning, T>(a, L, span_heads(a, target), target, stream, name);
+      const int64_t target = tile_words<T>(512, words);  // 2 a thread
+      const int64_t heads = span_heads(a, target);
+      if (heads * 2 * W <= 512 || words / (heads * 2 * W) >= 2 * kCUs)
+        return launch_tiles<D, I, kSpanning, T>(a, L, heads, target, stream, name);
     }
     return launch_tiles<D, I, kPlain, T>(a, L, EVS_SCATTER_HEADS_PER_TILE,
-                                        EVS_SCATTER_TILE_WORDS * kNarrow, stream, name);
+                                        tile_words<T>(EVS_SCATTER_TILE_WORDS, words), stream, name);
   }
 }
 

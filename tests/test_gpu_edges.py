@@ -196,6 +196,53 @@ def test_head_groups_of_every_tile_shape(ext, layout, heads_total, dtype, d, n):
             assert np.array_equal(bits(g), bits(w))
 
 
+# narrow words by width: 8, 4, 2 and 1 bytes, and 2 bytes of one element each
+NARROW = [(torch.float8_e4m3fn, 120, 8), (torch.float8_e4m3fn, 100, 4),
+          (torch.float8_e4m3fn, 126, 2), (torch.float8_e4m3fn, 121, 1), (torch.bfloat16, 121, 2)]
+
+
+@pytest.mark.parametrize("dtype,d,word", NARROW)
+@pytest.mark.parametrize("words", [1 << 18, 1 << 19, 1 << 21])
+def test_calls_past_the_sizes_at_which_tiles_grow(ext, dtype, d, word, words):
+    """Calls just past 2^18, 2^19 and 2^21 words, where the tiles of narrow words (and the head
+    groups of the gather's) change, by every kind of call, in kv_first and the combined layout."""
+    n_layers, heads, e = 2, [3, 0, 7, 1, 6, 2, 5, 4], 1 if dtype is torch.float8_e4m3fn else 2
+    n = words // (n_layers * len(heads) * 2 * (d * e // word)) + 3
+    nb = -(-n // BS) + 5
+    rng = np.random.default_rng(words + d)
+    starts = np.sort(rng.permutation(nb)[:-(-n // BS)]) * BS
+    ranged = (starts[:, None] + np.arange(BS)).reshape(-1)[:n]
+    slots = rng.permutation(nb * BS)[:n]
+    slots[rng.random(n) < 0.05] = -1
+    first = np.minimum(np.arange(starts.size + 1) * BS, n)
+    for layout in ("kv_first", "combined"):
+        layers = caches(layout, d, dtype, n_layers=n_layers, nb=nb, h=8, seed=d)
+        st = strides_of(layers[0])
+        want = oracle.gather_rows(layers, slots, heads, n, d, BS, st, e)
+        gpu = [t.cuda() for t in layers]
+        out = torch.zeros(want.nbytes, dtype=torch.uint8, device="cuda")
+        ext.gather_rows(ptrs(gpu), dev_long(slots), dev_long(heads), out.data_ptr(), n, d, BS,
+                        list(st), e)
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy().view(want.dtype).reshape(want.shape), want)
+        for kind in ("slots", "pairs", "ranges"):
+            dst = [torch.zeros_like(t) for t in layers]
+            gpu = [t.cuda() for t in dst]
+            args = (dev_long(heads), out.data_ptr(), n, d, BS, list(st), e)
+            if kind == "slots":
+                oracle.scatter_rows(dst, slots, heads, want, n, d, BS, st, e)
+                ext.scatter_rows(ptrs(gpu), dev_long(slots), *args)
+            elif kind == "pairs":
+                oracle.scatter_rows(dst, slots, heads, want[:, :, ::-1].copy(), n, d, BS, st, e)
+                ext.scatter_pairs(ptrs(gpu), dev_long(slots), dev_long(range(n - 1, -1, -1)), *args)
+            else:
+                oracle.scatter_rows(dst, ranged, heads, want, n, d, BS, st, e)
+                ext.scatter_ranges(ptrs(gpu), dev_long(starts), dev_long(first), n, *args)
+            torch.cuda.synchronize()
+            for g, w in zip(gpu, dst):
+                assert np.array_equal(bits(g), bits(w)), (layout, kind)
+
+
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("blocks", [[3], [9, 0, 77], list(range(40, 57))])
 def test_ragged_block_lists(ext, layout, blocks):
