@@ -808,14 +808,16 @@ int64_t span_heads(const RowsArgs& a, int64_t target) {
 // Sizes of a call, in words, at which its tiles change: below them a larger tile leaves a CU so
 // few waves that their own round trips are the call's time. From kTwice on the tiles of narrow
 // words hold twice a 16-byte word's number, from kFourTimes (words below 8 bytes) four times.
-// Below kFewWords a gather's tile has two heads at most. Microseconds with the large tiles at
-// every size, and so: gathers of 8 slots of 8 heads of one layer, fp8 120 3.85 and 2.64, bf16 120
-// 3.32 and 2.62; 16 slots x 32 layers 4.22 and 2.81, 3.60 and 2.85; the scatter's 8 slots of 8 fp8
-// heads of 120 3.12 and 2.66. Calls past each line ran as fast or faster in the larger tiles (0.4
-// to 3.5 million words of every width, each 1x, 2x and 4x).
+// Below kFewWords a gather's tile has two heads at most. From kHalfTile on the gather of kSmall's
+// rule takes half-size tiles. Microseconds with the large tiles at every size, and so: gathers of
+// 8 slots of 8 heads of one layer, fp8 120 3.85 and 2.64, bf16 120 3.32 and 2.62; 16 slots x 32
+// layers 4.22 and 2.81, 3.60 and 2.85; the scatter's 8 slots of 8 fp8 heads of 120 3.12 and 2.66.
+// Calls past each line ran as fast or faster in the larger tiles (0.4 to 3.5 million words of
+// every width, each 1x, 2x and 4x).
 constexpr int64_t kFewWords = 1024 * kCUs;
 constexpr int64_t kTwice = 2048 * kCUs;
 constexpr int64_t kFourTimes = 8192 * kCUs;
+constexpr int64_t kHalfTile = 65536 * kCUs;
 
 // The words a tile aims at in a call of `words`, with `base` a 16-byte word's.
 template <typename T>
@@ -836,11 +838,15 @@ int launch_typed(RowsArgs a, int64_t L, uint32_t W, hipStream_t stream, const ch
     const int64_t target = tile_words<T>(EVS_GATHER_TILE_WORDS, words);
     const int64_t hg = words < kFewWords ? EVS_GATHER_HEADS_PER_TILE : gather_heads(a, target);
     if constexpr (sizeof(T) == 16) {
-      // Two heads a tile of several (their rows far apart, see gather_heads), in whole lines: half
-      // the tile. bf16 heads of 128, 32 layers, 8 heads: 16,384 slots 6,179 against 6,168 GB/s,
-      // 32,768 5,986 against 5,912; 4 heads of 64, 32,768 6,183 against 6,157. Four heads a tile,
-      // one head and the combined layout gained nothing from it.
-      if (hg == 2 && a.H > 2 && a.sh == a.half_bytes && per_line(a.half_bytes) == 1)
+      // Two heads a tile of several (their rows far apart, see gather_heads), half-rows of one or
+      // two whole lines, in a large call: half the tile. bf16 heads of 128, microseconds a call in
+      // half-size and whole tiles: 8 heads, 16,384 slots x 32 layers 706 and 711, 32,768 x 16 760
+      // and 770; 4 heads, 32,768 x 16 363 and 370; 16 heads, 32,768 x 16 1,588 and 1,581; d 64 the
+      // same within 1 %. Half-rows of 512 bytes lost (8 heads, 32,768 x 16 1,543 and 1,471), and so
+      // did smaller calls (4 heads, 1,000 slots x 32 layers 24.5 and 22.9; 8 32-bit heads, 1,500
+      // slots of one layer 6.6 and 5.4).
+      if (hg == 2 && a.H > 2 && a.sh == a.half_bytes && per_line(a.half_bytes) == 1 &&
+          a.half_bytes <= 256 && words >= kHalfTile)
         return launch_tiles<D, I, kSmall, T>(a, L, hg, target / 2, stream, name);
     }
     return launch_tiles<D, I, kPlain, T>(a, L, hg, target, stream, name);

@@ -243,6 +243,20 @@ def test_calls_past_the_sizes_at_which_tiles_grow(ext, dtype, d, word, words):
                 assert np.array_equal(bits(g), bits(w)), (layout, kind)
 
 
+def test_a_gather_past_the_size_at_which_its_tiles_halve(ext):
+    """2^24 16-byte words of heads whose staged rows lie far apart, against torch's indexing."""
+    n_layers, h, n, d, nb = 8, 8, 8200, 128, 2100
+    g = torch.Generator(device="cuda").manual_seed(3)
+    layers = [torch.randint(-(1 << 15), 1 << 15, (2, nb, BS, h, d), generator=g, device="cuda",
+                            dtype=torch.int16) for _ in range(n_layers)]
+    slots = torch.randperm(nb * BS, generator=g, device="cuda")[:n]
+    out = torch.zeros((n_layers, h, n, 2, d), dtype=torch.int16, device="cuda")
+    ext.gather_rows(ptrs(layers), slots, dev_long(range(h)), out.data_ptr(), n, d, BS,
+                    [BS * h * d, h * d, d, nb * BS * h * d, 1], 2)
+    for layer, rows in zip(layers, out):
+        assert torch.equal(rows, layer.view(2, nb * BS, h, d)[:, slots].permute(2, 1, 0, 3))
+
+
 @pytest.mark.parametrize("layout", LAYOUTS)
 @pytest.mark.parametrize("blocks", [[3], [9, 0, 77], list(range(40, 57))])
 def test_ragged_block_lists(ext, layout, blocks):
