@@ -96,7 +96,7 @@ constexpr int kVectors = 1;        // mode bit: every member buffer 16-byte alig
 constexpr int kEarly = 2;          // mode bit: early start (a member missing at the first read)
 constexpr int kFew = 4;            // mode bit: at most kFewMembers listed, and vectors to move
 constexpr int kFewMembers = 4;
-constexpr int kFewPasses = 8;
+constexpr int kFewPasses = 2;       // a call of kFewMembers longer than this takes single passes
 constexpr int kDoneBits = 20;      // counting words: workgroups done in bits [0, 20), outcome above
 constexpr uint32_t kGroups = 8;    // group counting words
 // Grids up to this many workgroups count flat, into the top word: their atomics on one address
@@ -535,9 +535,11 @@ __global__ __launch_bounds__(kBlockThreads + 64) void local_reduce(ReduceArgs a)
   // the widest kernel then takes several passes at once, in the same registers. Microseconds a
   // call, one pass at a time and now: two members of 1,200,000 elements 5.67 and 4.48, 3,000,000
   // 8.68 and 6.37, 33,000,000 49.8 and 36.3; three of 33,000,000 52.2 and 46.1; four of 3,000,000
-  // 9.59 and 8.14. Four members fill the memory's rate by themselves in a long call (33,554,432
-  // elements: 57.2, 57.8 in groups), and take single passes past kFewPasses, of four members'
-  // loads instead of eight (20,000,000 elements 36.9 and 35.9, 33,554,432 58.0 and 57.7).
+  // 8.76 and 7.14. Four members gain from two passes at once only while a workgroup has no more
+  // than two (2,200,000 elements 6.76, 7.15 one at a time; 4,194,304 7.91 and 8.18; 8,000,000 14.5
+  // and 13.6; 16,777,216 28.7 and 28.1); past them they take single passes, of four members' loads
+  // instead of eight (8,000,000 elements 15.8 and 13.6, 20,000,000 34.8 and 33.7, 33,554,432, where
+  // the memory's rate bounds both, 55.2 and 55.3).
   constexpr bool kTakesFew = kControl && EVS_REDUCE_FENCE == 3 && V == kMaxVpt && V > 1;
   __shared__ const uint16_t* s_src[kMaxRows];  // member in order position q, or null: missing
   __shared__ int s_count;
