@@ -457,8 +457,9 @@ class Kernels:
         device and stream), or in staged order (``evs_scatter_rows``, one kernel). The same bytes
         land either way. ``None`` sorts from :data:`ORDER_MIN_SLOTS` slots and
         :data:`ORDER_MIN_BYTES` of rows, where writing a whole cache through a permuted block
-        table in slot order repays the sort, and never under graph capture (the sort clears its
-        counters with a memset, which a captured graph must not hold). ``num_slots``, the
+        table in slot order repays the sort, and never under graph capture (the sort's workspace is
+        the one eager calls on the stream use and replace, and above 2^20 pairs it clears counters
+        with a memset, which a captured graph must not hold). ``num_slots``, the
         caches' slot count when the caller knows it, lets that choice see how much of the cache
         the call writes (:func:`sort_first`).
         """
@@ -478,7 +479,8 @@ class Kernels:
                 ordered = sort_first(n, nl, nh, int(d), int(elem_size), capturing, num_slots)
             if ordered and capturing:
                 raise RuntimeError("scatter_rows: an ordered scatter cannot be captured in a graph "
-                                   "(its sort clears counters with a memset)")
+                                   "(its sort uses the stream's shared workspace, and above 2^20 "
+                                   "pairs a memset)")
             if not ordered:
                 self._check(
                     self._lib.evs_scatter_rows(
