@@ -18,9 +18,12 @@
 // 22.4 and 44.4, 262,144 29.8 and 106.4 (32 bits: 37.0 and 107.9); 21 bits, 1,048,576 pairs: 75
 // and 191.
 // Above 2^20 pairs rocPRIM's radix sort is used (2,097,152 pairs of 21 bits: 120 us, 197 here):
-// every workgroup adds up every tile's counts, work that grows with the square of the tiles.
-// rocPRIM clears its counters in the workspace with hipMemsetAsync, so this call is not one to
-// capture in a HIP graph.
+// every workgroup adds up every tile's counts, work that grows with the square of the tiles. So it
+// is for a few sizes below (see kMergedFirst). Slower here than there are left ids that need more
+// than two passes of up to 4,000 pairs (20 bits: TINYFIG) and ids that need four and more passes of up
+// to 36,000 (32 bits: 43.4 against 40.9 us at 32,768; 64 bits, up to 200,000: 103 against 80).
+// Padding ids need every pass of their key. rocPRIM clears its counters in the workspace with
+// hipMemsetAsync, so this call is not one to capture in a HIP graph.
 //
 // evs_order_pairs_static is the same call for callers that cannot allocate (no workspace
 // argument): its scratch is a file-scope device array of a fixed size.
@@ -54,9 +57,17 @@ int rounds_of(int64_t n) { return n <= kMaxTiles * tile_pairs(4) ? 4 : 8; }
 static_assert(kMaxTiles * tile_pairs(8) >= kMaxSorted && tile_pairs(8) < 65536,
               "a tile's counts are 16 bits");
 // Up to this many pairs one workgroup sorts them all in one launch: 5,000 in 16.5 us, 19.1 in four
-// launches (18 bits); kHalfTile and fewer in a smaller one.
+// launches (18 bits); kHalfTile and kQuarterTile and fewer in smaller ones.
 constexpr int64_t kOneTile = 8192;
-constexpr int64_t kHalfTile = 2048;
+constexpr int64_t kHalfTile = 4096;
+constexpr int64_t kQuarterTile = 2048;
+// From kOneTile to this many pairs, keys of three passes and more take rocPRIM's sort, which merges
+// once less often than above: 8,193 and 16,384 pairs of 20 bits 27.4 and 29.1 us (31.0 and 31.8
+// here), of 32 bits 29.5 and 30.1, here 28.1 and 28.9 for ids of 18 bits and 41.5 and 42.7 with
+// padding among them; 20,000 pairs of 20 bits 38.3 (32.0).
+constexpr int64_t kMergedFirst = 16384;
+// A workspace that holds that sort's, for every larger call of such keys too.
+constexpr int64_t kMergedBytes = int64_t{512} << 10;
 
 struct SortArgs {
   const int64_t* slots;  // the ids as given
@@ -385,6 +396,12 @@ bool overlap(const void* p, int64_t p_bytes, const void* q, int64_t q_bytes) {
   return x < y + static_cast<uintptr_t>(q_bytes) && y < x + static_cast<uintptr_t>(p_bytes);
 }
 
+// Whether an output overlaps the ids.
+bool writes_ids(const int64_t* slots, int64_t n, const int64_t* slots_out,
+                const int64_t* rows_out) {
+  return overlap(slots, n * 8, slots_out, n * 8) || overlap(slots, n * 8, rows_out, n * 8);
+}
+
 int tiles_of(int64_t n) {
   const int64_t tile = tile_pairs(rounds_of(n));
   return static_cast<int>((n + tile - 1) / tile);
@@ -396,6 +413,13 @@ int tiles_of(int64_t n) {
 int64_t sorted_bytes(int64_t n) {
   const int64_t tiles = (n + tile_pairs(4) - 1) / tile_pairs(4);
   return 2 * round_up(n * 8) + round_up(tiles * kBins * 2) + round_up(tiles * 8);
+}
+
+// Whether the radix sort takes these pairs (where an output overlaps the ids it takes every call of
+// up to kMaxSorted).
+bool sorted_here(int64_t n, int bits) {
+  const bool merged = n > kOneTile && n <= kMergedFirst && bits > 2 * kDigitBits;
+  return n <= kMaxSorted && !merged;
 }
 
 int sort_pairs(const int64_t* slots, int64_t n, int bits, int64_t* slots_out, int64_t* rows_out,
@@ -415,16 +439,16 @@ int sort_pairs(const int64_t* slots, int64_t n, int bits, int64_t* slots_out, in
   w += round_up(int64_t{a.tiles} * kBins * 2);
   a.ors = reinterpret_cast<uint64_t*>(w);
   a.key_mask = bits == 64 ? ~uint64_t{0} : (uint64_t{1} << bits) - 1;
-  a.even = overlap(slots, n * 8, slots_out, n * 8) || overlap(slots, n * 8, rows_out, n * 8);
+  a.even = writes_ids(slots, n, slots_out, rows_out);
   const dim3 threads(kSortThreads);
   // one workgroup reads every id before it writes: an overlap is no matter
-  if (n <= kHalfTile) {
-    hipLaunchKernelGGL((sort_tile<512, 4>), dim3(1), dim3(512), 0, s, a);
-    EVS_LAUNCHED("evs_order_pairs");
-    return EVS_OK;
-  }
   if (n <= kOneTile) {
-    hipLaunchKernelGGL((sort_tile<1024, 8>), dim3(1), dim3(1024), 0, s, a);
+    if (n <= kQuarterTile)
+      hipLaunchKernelGGL((sort_tile<512, 4>), dim3(1), dim3(512), 0, s, a);
+    else if (n <= kHalfTile)
+      hipLaunchKernelGGL((sort_tile<1024, 4>), dim3(1), dim3(1024), 0, s, a);
+    else
+      hipLaunchKernelGGL((sort_tile<1024, 8>), dim3(1), dim3(1024), 0, s, a);
     EVS_LAUNCHED("evs_order_pairs");
     return EVS_OK;
   }
@@ -495,6 +519,8 @@ extern "C" int evs_order_pairs_workspace(int64_t num_pairs, int key_bits, int64_
   EVS_REQUIRE(key_bits >= 1 && key_bits <= 64, "evs_order_pairs_workspace: key_bits in 1..64");
   if (num_pairs <= evs::kMaxSorted) {
     *bytes = evs::sorted_bytes(num_pairs);
+    const bool merged = num_pairs > evs::kOneTile && key_bits > 2 * evs::kDigitBits;
+    if (merged && *bytes < evs::kMergedBytes) *bytes = evs::kMergedBytes;
     return EVS_OK;
   }
   size_t sort_bytes = 0;
@@ -509,7 +535,7 @@ extern "C" int evs_order_pairs(const int64_t* slots, int64_t num_pairs, int key_
                                int64_t workspace_bytes, void* stream) {
   evs::clear_error();
   int64_t need = 0;
-  const int rc = evs_order_pairs_workspace(num_pairs, key_bits, &need);
+  int rc = evs_order_pairs_workspace(num_pairs, key_bits, &need);
   if (rc != EVS_OK) return rc;
   if (num_pairs == 0) return EVS_OK;
   EVS_REQUIRE(slots != nullptr && slots_out != nullptr && rows_out != nullptr &&
@@ -522,11 +548,18 @@ extern "C" int evs_order_pairs(const int64_t* slots, int64_t num_pairs, int key_
               "evs_order_pairs: the workspace must be %lld-byte aligned",
               static_cast<long long>(evs::kAlign));
   hipStream_t s = evs::as_stream(stream);
-  if (num_pairs <= evs::kMaxSorted)
+  const bool in_place = num_pairs <= evs::kMaxSorted &&
+                        evs::writes_ids(slots, num_pairs, slots_out, rows_out);
+  if (evs::sorted_here(num_pairs, key_bits) || in_place)
     return evs::sort_pairs(slots, num_pairs, key_bits, slots_out, rows_out, workspace, s);
   int64_t* rows = static_cast<int64_t*>(workspace);
   char* sort_tmp = static_cast<char*>(workspace) + evs::round_up(num_pairs * 8);
-  size_t sort_bytes = static_cast<size_t>(need - evs::round_up(num_pairs * 8));
+  size_t sort_bytes = 0;
+  rc = evs::sort_storage(num_pairs, key_bits, &sort_bytes);
+  if (rc != EVS_OK) return rc;
+  EVS_REQUIRE(evs::round_up(num_pairs * 8) + static_cast<int64_t>(sort_bytes) <= need,
+              "evs_order_pairs: rocPRIM needs %lld bytes for %lld pairs",
+              static_cast<long long>(sort_bytes), static_cast<long long>(num_pairs));
   const int64_t grid = (num_pairs + evs::kIotaThreads - 1) / evs::kIotaThreads;
   hipLaunchKernelGGL(evs::iota, dim3(static_cast<uint32_t>(grid)), dim3(evs::kIotaThreads), 0, s,
                      rows, num_pairs);

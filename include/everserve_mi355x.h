@@ -144,9 +144,11 @@ int evs_scatter_ranges(const int64_t* layer_ptrs, int64_t num_layers, const int6
  * slot id (padding) lands wherever its low bits put it, and evs_scatter_pairs skips it.
  * `workspace` is device memory of at least evs_order_pairs_workspace(num_pairs, key_bits) bytes,
  * 256-byte aligned, owned by the caller; the call allocates nothing and does not synchronise.
- * Above 2^20 pairs the sort clears its own counters in the workspace with hipMemsetAsync, so keep
- * this call out of captured HIP graphs. num_pairs < 2^31. No counterpart in the reference: it orders the restore's writes (see
- * evs_scatter_pairs); the host-side equivalent is everserve_amd.state.restore.destination_order. */
+ * The workspace grows with num_pairs, so that a call's serves smaller ones of the same key_bits.
+ * For some sizes, all above 2^20 pairs among them, the sort clears counters in the workspace with
+ * hipMemsetAsync, so keep this call out of captured HIP graphs. num_pairs < 2^31. No counterpart in
+ * the reference: it orders the restore's writes (see evs_scatter_pairs); the host-side equivalent is
+ * everserve_amd.state.restore.destination_order. */
 int evs_order_pairs_workspace(int64_t num_pairs, int key_bits, int64_t* bytes);
 int evs_order_pairs(const int64_t* slots, int64_t num_pairs, int key_bits, int64_t* slots_out,
                     int64_t* rows_out, void* workspace, int64_t workspace_bytes, void* stream);

@@ -146,11 +146,11 @@ def test_scatter_rows_sorts_first_from_two_to_the_18_slots_and_8_gib():
     assert not sf((7 << 17) - 1, capturing=False, num_slots=1 << 20, **c4)
 
 
-@pytest.mark.parametrize("bits", [1, 18, 64])
+@pytest.mark.parametrize("bits", [1, 18, 19, 64])
 def test_the_orders_workspace_grows_with_the_pairs(lib, bits):
     """A caller that sizes the workspace for its largest call may use it for every smaller one:
     the bytes never fall as the pairs grow, over each place where the sort changes its tiles."""
-    edges = [2048, 8192, 1 << 18, 1 << 19, 532_384, 1 << 20]
+    edges = [2048, 8192, 16_384, 1 << 18, 1 << 19, 532_384, 1 << 20]
     sizes = sorted({0, 1, *(e + d for e in edges for d in range(-3, 4)), *range(1, 1 << 20, 4099)})
     sizes = [n for n in sizes if n <= 1 << 20]  # past it the sort asks the device
     need, got = ctypes.c_int64(), []

@@ -6,6 +6,8 @@ for each, ties in listed order. Then ordering on the device and scattering the p
 the same caches as the scatter in staged order.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -69,6 +71,42 @@ def test_the_ids_sorted_where_they_lie(ext, n, bits):
     want = np.argsort(slots, kind="stable")
     assert np.array_equal(rows.cpu().numpy(), want)
     assert np.array_equal(dev.cpu().numpy(), slots[want])
+
+
+@pytest.mark.parametrize("n", [4096, 4097, 16_384, 16_385])
+@pytest.mark.parametrize("bits", [18, 19, 32])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_the_sizes_between_the_sorts(ext, n, bits, in_place):
+    """One workgroup's smaller sort, and the sizes from which and up to which keys of three passes
+    take rocPRIM's sort unless their ids are sorted where they lie, in the workspace a C caller
+    sizes for that very call."""
+    rng = np.random.default_rng(n + bits)
+    slots = rng.integers(0, 1 << min(bits, 20), n)
+    slots[rng.random(n) < 0.01] = -1
+    low = slots.astype(np.uint64) & np.uint64((1 << bits) - 1)
+    want = np.argsort(low, kind="stable")
+    dev = torch.from_numpy(slots.copy()).cuda()
+    keys = dev if in_place else torch.empty_like(dev)
+    rows = torch.empty_like(dev)
+    need = ctypes.c_int64()
+    assert ext._lib.evs_order_pairs_workspace(n, bits, ctypes.byref(need)) == 0
+    work = torch.empty(need.value, dtype=torch.uint8, device="cuda")
+    assert ext._lib.evs_order_pairs(dev.data_ptr(), n, bits, keys.data_ptr(), rows.data_ptr(),
+                                    work.data_ptr(), need.value,
+                                    torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(rows.cpu().numpy(), want)
+    assert np.array_equal(keys.cpu().numpy(), slots[want])
+
+
+@pytest.mark.parametrize("bits", [18, 21, 64])
+def test_the_workspace_grows_past_the_radix_sort(ext, bits):
+    """Over the size at which rocPRIM's sort takes over, whose storage the device is asked for."""
+    need, got = ctypes.c_int64(), []
+    for n in (1 << 20, (1 << 20) + 1, (1 << 20) + 70_000, 1 << 21):
+        assert ext._lib.evs_order_pairs_workspace(n, bits, ctypes.byref(need)) == 0
+        got.append(need.value)
+    assert got == sorted(got)
 
 
 def test_ties_keep_their_listed_order(ext):
