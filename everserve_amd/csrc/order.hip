@@ -19,11 +19,10 @@
 // and 191.
 // Above 2^20 pairs rocPRIM's radix sort is used (2,097,152 pairs of 21 bits: 120 us, 197 here):
 // every workgroup adds up every tile's counts, work that grows with the square of the tiles. So it
-// is for a few sizes below (see kMergedFirst). Slower here than there are left ids that need more
-// than two passes of up to 4,000 pairs (20 bits: TINYFIG) and ids that need four and more passes of up
-// to 36,000 (32 bits: 43.4 against 40.9 us at 32,768; 64 bits, up to 200,000: 103 against 80).
-// Padding ids need every pass of their key. rocPRIM clears its counters in the workspace with
-// hipMemsetAsync, so this call is not one to capture in a HIP graph.
+// is for a few sizes below (see kMergedFirst). Left slower here than there: ids that need all four
+// passes of a 32-bit key, up to 36,000 pairs (32,768 pairs 43.4 and 40.9 us), and more passes, up
+// to 200,000 (64 bits 103 and 80); padding ids need every pass of their key. rocPRIM clears its
+// counters in the workspace with hipMemsetAsync, so this call is not one to capture in a HIP graph.
 //
 // evs_order_pairs_static is the same call for callers that cannot allocate (no workspace
 // argument): its scratch is a file-scope device array of a fixed size.
@@ -57,7 +56,8 @@ int rounds_of(int64_t n) { return n <= kMaxTiles * tile_pairs(4) ? 4 : 8; }
 static_assert(kMaxTiles * tile_pairs(8) >= kMaxSorted && tile_pairs(8) < 65536,
               "a tile's counts are 16 bits");
 // Up to this many pairs one workgroup sorts them all in one launch: 5,000 in 16.5 us, 19.1 in four
-// launches (18 bits); kHalfTile and kQuarterTile and fewer in smaller ones.
+// launches (18 bits). kHalfTile and fewer take half its rounds (2,049 pairs of 18 bits 10.6 and 15.0
+// us, 4,000 of 20 bits 14.9 and 20.6), kQuarterTile and fewer half the waves too.
 constexpr int64_t kOneTile = 8192;
 constexpr int64_t kHalfTile = 4096;
 constexpr int64_t kQuarterTile = 2048;
