@@ -52,10 +52,12 @@ REDUCE_STATE_WORDS = 288
 ORDER_MIN_SLOTS = 1 << 18
 ORDER_MIN_BYTES = 8 << 30
 """The sizes from which :meth:`Kernels.scatter_rows` sorts its pairs by slot first. Measured on
-MI355X (Llama-3-8B rows, bf16, 16-slot blocks of a permuted table, median of 10 launches), sorted
-against staged order, a sort of 0.11 ms included (0.04 since): every slot of a 262,144-slot cache, 32 layers,
-11.58 against 12.17 ms; 8 layers 2.86 against 3.02; 4 layers 1.52 against 1.53; 1 layer 0.47
-against 0.38 (the sort not repaid); a quarter of the cache's blocks, 32 layers, 3.12 against 3.08
+MI355X (Llama-3-8B rows, bf16, 16-slot blocks of a permuted table, median of 9 launches), sorted
+against staged order, a sort of 0.04 ms included: every slot of a 262,144-slot cache, 32 layers,
+11.52 against 12.15 ms; 8 layers (8 GiB) 2.94 against 3.04; 4 layers 1.50 against 1.53; 2 layers
+0.77 against 0.76; 1 layer 0.42 against 0.39 (the sort not repaid). The line is where the order is
+worth 3 % and more; from 3 GiB on ``ordered=True`` gains 1.6 % of such a call. A quarter of the
+cache's blocks, 32 layers, 3.12 against 3.08 with a sort of 0.11 ms
 (writes spread over a sparse part of a cache gain nothing from order). The call cannot see the
 cache's size unless told it (``num_slots``), so a call of this many slots into a cache several
 times larger sorts too, and can lose up to about 3 %: pass ``num_slots`` or ``ordered=False``
