@@ -272,7 +272,7 @@ using global_ptr = __attribute__((address_space(1))) T*;
 // instructions are the aligned ones). Microseconds a call where the bases lie one element off the
 // word, moved by elements, by words cut into bytes and so: the gather of 8,192 slots of one
 // bf16 head of 100, 32 layers, 177, 114 and 46; of one 32-bit head of 126 197, 310 and 95; of 8
-// slots of 8 bf16 heads of 100, one layer, 2.9, 9.6 and 3.9.
+// slots of 8 bf16 heads of 100, one layer, 2.8, 9.6 and 3.1.
 enum Side : int { kStaged, kCache };
 template <typename T, Side S>
 struct WordOn {
